@@ -61,6 +61,18 @@ __device__ __forceinline__ void buffer_store(T x, __amdgpu_buffer_rsrc_t r, std:
     }
 }
 
+// A record at a wave-uniform address that no kernel in flight writes, through
+// the scalar cache (the constant address space): one scalar load, where a
+// plain load would go through vector registers, since the kernel's own stores
+// could alias it as far as the compiler knows.
+template <class T>
+__device__ __forceinline__ T constant_load(const T* p) {
+    using C = const __attribute__((address_space(4))) T;
+    T x;
+    __builtin_memcpy(&x, (C*)(p), sizeof(T));
+    return x;
+}
+
 // Wave-uniform copies (readfirstlane returns int: go through uint32 so the
 // low half of a 64-bit value is not sign-extended).
 __device__ __forceinline__ std::uint32_t uniform(std::uint32_t x) {

@@ -112,7 +112,7 @@ struct EngineImplT {
     bool lazy = false;
     int arith = kStrict;
     std::uint32_t l1 = 0, l2 = 0;
-    DeviceBuffer tables, domains, poly_domain, in_off, out_off;
+    DeviceBuffer tables, poly_domains, in_off, out_off;
     struct Launch {
         PassLaunch<W> fn;
         unsigned grid;
@@ -137,21 +137,24 @@ struct EngineImplT {
         const std::uint64_t polys = c.polynomials.empty() ? c.batch : c.polynomials.size();
         require(polys >= 1 && polys <= 0xffffffffull, "NTT batch must be in [1, 2^32)");
         const bool offsets = !c.polynomials.empty();
-        if (offsets) {
-            std::vector<std::uint32_t> pd;
-            std::vector<std::uint64_t> io, oo;
-            for (const auto& p : c.polynomials) {
-                pd.push_back(p.domain);
-                io.push_back(p.input_offset);
-                oo.push_back(p.output_offset);
-            }
-            poly_domain.upload(pd);
-            in_off.upload(io);
-            out_off.upload(oo);
-        }
+        PassArgs<W> in_args{}, out_args{};  // the caller's sides: offsets of the first and last pass
+        place(c, &NttPolynomial::input_offset, in_off, in_args.in_base, in_args.in_step, in_args.in_off);
+        place(c, &NttPolynomial::output_offset, out_off, out_args.out_base, out_args.out_step, out_args.out_off);
         const bool mixed = c.domains.size() > 1;
         PassArgs<W> base{};
         base.polys = static_cast<std::uint32_t>(polys);
+        base.in_step = base.out_step = n;  // packed rows (the workspace side of two-pass plans)
+        const auto input_side = [&](PassArgs<W>& a) {
+            a.in_base = in_args.in_base;
+            a.in_step = in_args.in_step;
+            a.in_off = in_args.in_off;
+            a.reduce_input = c.reduce_input;
+        };
+        const auto output_side = [&](PassArgs<W>& a) {
+            a.out_base = out_args.out_base;
+            a.out_step = out_args.out_step;
+            a.out_off = out_args.out_off;
+        };
         constexpr int LB = kTileLog;
         const bool ct = !c.inverse;
         // Which physical boundaries differ from the algorithm's native order
@@ -172,9 +175,8 @@ struct EngineImplT {
             L.grid = unsigned(tiles);
             L.args = base;
             L.args.tiles = unsigned(tiles);
-            L.args.in_off = in_off.as<std::uint64_t>();
-            L.args.out_off = out_off.as<std::uint64_t>();
-            L.args.reduce_input = c.reduce_input;
+            input_side(L.args);
+            output_side(L.args);
             L.lt = int(log_n);
             L.prefix_bits = 0;
             L.last = true;
@@ -212,18 +214,16 @@ struct EngineImplT {
             B.fn = find_pass<W>(
                 PassKey{arith, int(log_n), int(l2), rli, false, ct, !ct && perm_in, ct && perm_out, false});
             if (ct) {  // forward: A reads the input, B writes the output
-                A.args.in_off = in_off.as<std::uint64_t>();
-                A.args.reduce_input = c.reduce_input;
+                input_side(A.args);
                 A.writes_workspace = true;
                 B.reads_workspace = true;
-                B.args.out_off = out_off.as<std::uint64_t>();
+                output_side(B.args);
                 launches = {A, B};
             } else {  // inverse: B reads the input, A writes the output
-                B.args.in_off = in_off.as<std::uint64_t>();
-                B.args.reduce_input = c.reduce_input;
+                input_side(B.args);
                 B.writes_workspace = true;
                 A.reads_workspace = true;
-                A.args.out_off = out_off.as<std::uint64_t>();
+                output_side(A.args);
                 launches = {B, A};
             }
             json_shape = "{\"passes\":2,\"high_bits\":" + std::to_string(l1) + ",\"low_bits\":" +
@@ -234,6 +234,28 @@ struct EngineImplT {
         // domains, so the phase offsets are shared).
         if (arith == kBarrett) build_tables<W>(c, n, ct);
         else build_tables<TwPair<W>>(c, n, ct);
+    }
+
+    // Word offsets of the polynomials on one side: base + p * step where they
+    // form such a sequence (packed, pitched and dense RNS rows: no table to
+    // read before the first data load), else a device table.
+    void place(const NttEngineConfig& c, std::uint64_t NttPolynomial::*side, DeviceBuffer& table, std::uint64_t& base,
+               std::uint64_t& step, const std::uint64_t*& off) {
+        base = 0;
+        step = std::uint64_t{1} << c.log_n;
+        off = nullptr;
+        const auto& ps = c.polynomials;
+        if (ps.empty()) return;
+        base = ps[0].*side;
+        step = ps.size() > 1 ? ps[1].*side - base : 0;  // modulo 2^64, as the kernel's sum
+        bool sequence = true;
+        for (std::size_t i = 0; i < ps.size() && sequence; ++i) sequence = ps[i].*side == base + i * step;
+        if (sequence) return;
+        std::vector<std::uint64_t> host;
+        host.reserve(ps.size());
+        for (const auto& p : ps) host.push_back(p.*side);
+        table.upload(host);
+        off = table.as<std::uint64_t>();
     }
 
     // Entry E: a Shoup pair, or the bare twiddle word (Barrett).
@@ -276,13 +298,18 @@ struct EngineImplT {
         }
         require(all_tables.size() * sizeof(E) < 0x7fffffffull, "NTT twiddle tables exceed 2 GiB");
         tables.upload(all_tables);
-        domains.upload(host_domains);
+        if (host_domains.size() > 1) {
+            std::vector<DeviceDomain<W>> records;
+            records.reserve(c.polynomials.size());
+            for (const auto& p : c.polynomials) records.push_back(host_domains[p.domain]);
+            poly_domains.upload(records);
+        }
         const std::size_t per_domain = all_tables.size() / c.domains.size();
         for (auto& L : launches) {
             L.args.tw_bytes = static_cast<std::uint32_t>(per_domain * sizeof(E));
-            L.args.domains = domains.as<DeviceDomain<W>>();
+            L.args.domain = host_domains[0];
+            L.args.poly_domains = poly_domains.as<DeviceDomain<W>>();
             L.args.tw = tables.as<E>();
-            L.args.poly_domain = poly_domain.as<std::uint32_t>();
         }
     }
 

@@ -70,10 +70,15 @@ template <class W>
 struct PassArgs {
     const W* in;
     W* out;
-    const DeviceDomain<W>* domains;
-    const void* tw;                    // all domains' chunk tables (Entry), concatenated
-    const std::uint32_t* poly_domain;  // per polynomial (null: domain 0)
-    const std::uint64_t* in_off;       // per polynomial word offset (null: p << log n)
+    const void* tw;  // all domains' chunk tables (Entry), concatenated
+    // The domain, in the kernel arguments where all polynomials share one;
+    // else one record per polynomial (a single dependent scalar load).
+    DeviceDomain<W> domain;
+    const DeviceDomain<W>* poly_domains;
+    // Polynomial p starts at word in_base + p * in_step of the input, or at
+    // in_off[p] where the offsets are no such sequence; the output likewise.
+    std::uint64_t in_base, in_step, out_base, out_step;
+    const std::uint64_t* in_off;
     const std::uint64_t* out_off;
     std::uint32_t polys, tiles;
     std::uint32_t reduce_input;
@@ -471,18 +476,12 @@ struct Pass {
         return tl;
     }
 
-    // Buffer over the tile's span: its polynomial (two-pass, or one-pass with
-    // explicit offsets, where a tile holds one polynomial) or its run of dense
-    // polynomials (one-pass).
-    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t span(const W* base, const std::uint64_t* off,
-                                                                  const Tile& tl) {
-        // Offsets are read back into scalar registers (see domain_of).
-        if constexpr (SINGLE) {
-            if (off) return make_rsrc(base + uniform(off[tl.poly]), kPolyBytes);
-            return make_rsrc(base + (std::uint64_t(tl.poly) << kLogN), tl.lines * kPolyBytes);
-        } else {
-            return make_rsrc(base + (off ? uniform(off[tl.poly]) : std::uint64_t(tl.poly) << kLogN), kPolyBytes);
-        }
+    // Buffer over the tile's span: its polynomial, or its run of dense
+    // polynomials (one-pass tiles of several).
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t span(const W* base, std::uint64_t first, std::uint64_t step,
+                                                                  const std::uint64_t* off, const Tile& tl) {
+        const std::uint64_t word = off ? constant_load(off + tl.poly) : first + tl.poly * step;
+        return make_rsrc(base + word, (SINGLE ? tl.lines : 1u) * kPolyBytes);
     }
 
     // Logical row of line rr in a ROW tile.
@@ -692,7 +691,7 @@ struct Pass {
     // happen in process()).
     static __device__ __forceinline__ void load_tile(const PassArgs<W>& a, const Tile& tl, std::uint32_t t,
                                                      W (&v)[kE]) {
-        const __amdgpu_buffer_rsrc_t src = span(a.in, a.in_off, tl);
+        const __amdgpu_buffer_rsrc_t src = span(a.in, a.in_base, a.in_step, a.in_off, tl);
         constexpr int S = tile_window<0>();
         constexpr std::uint32_t B = sizeof(W);
         const std::uint32_t tw = PIN ? staged_base(tl, t).word : thread_word<S>(tl, t);
@@ -754,7 +753,7 @@ struct Pass {
                 v[r] = csub(x, d.q);
             }
         }
-        const __amdgpu_buffer_rsrc_t dst = span(a.out, a.out_off, tl);
+        const __amdgpu_buffer_rsrc_t dst = span(a.out, a.out_base, a.out_step, a.out_off, tl);
         if constexpr (POUT) {
             lds_barrier();
 #pragma unroll
@@ -793,24 +792,12 @@ struct Pass {
         }
     }
 
-    // One domain per tile (the planner keeps mixed-domain tiles apart). The
-    // record is wave-uniform; it comes back through vector loads (the
-    // kernel's stores could alias it as far as the compiler knows), so each
-    // field is read back into a scalar register.
+    // One domain per tile (the planner keeps mixed-domain tiles apart). At
+    // kernel start every dependent load costs a trip past the L2 (about half
+    // a microsecond of a pass of 9-14 us), so the record is in the kernel
+    // arguments or one scalar load away, never behind an index table.
     static __device__ __forceinline__ DeviceDomain<W> domain_of(const PassArgs<W>& a, const Tile& tl) {
-        const std::uint32_t dom = a.poly_domain ? uniform(a.poly_domain[tl.poly]) : 0u;
-        const DeviceDomain<W> d = a.domains[dom];
-        DeviceDomain<W> u;
-        u.q = uniform(d.q);
-        u.q2 = uniform(d.q2);
-        u.nq = uniform(d.nq);
-        u.rwp = uniform(d.rwp);
-        u.ninv = {uniform(d.ninv.w), uniform(d.ninv.wp)};
-        u.last = {uniform(d.last.w), uniform(d.last.wp)};
-        u.mu = uniform(d.mu);
-        u.qbits = uniform(d.qbits);
-        u.tw = uniform(d.tw);
-        return u;
+        return a.poly_domains ? constant_load(a.poly_domains + tl.poly) : a.domain;
     }
 
     // One tile: its words, its twiddle chunks, the butterflies and the
