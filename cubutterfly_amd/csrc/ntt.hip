@@ -54,7 +54,11 @@ void ensure_registered() {
         register_u32_barrett();
         register_u64_barrett();
         register_alt_u32();
+        register_u64_headroom();
         register_alt_u64();
+        register_alt_u64_headroom();
+        register_long_rows_u32();
+        register_long_rows_u64();
         return true;
     }();
     (void)once;
@@ -128,12 +132,18 @@ struct EngineImplT {
         const std::uint32_t log_n = c.log_n;
         const std::uint64_t n = std::uint64_t{1} << log_n;
         const unsigned bits = sizeof(W) * 8;
-        std::uint64_t max_q = 0;
-        for (const auto& d : c.domains) max_q = std::max(max_q, d.modulus);
+        std::uint64_t max_q = 0, min_q = ~std::uint64_t{0};
+        for (const auto& d : c.domains) {
+            max_q = std::max(max_q, d.modulus);
+            min_q = std::min(min_q, d.modulus);
+        }
         lazy = !c.force_strict && !c.barrett && max_q < (std::uint64_t{1} << (bits - 2));
         supported(!c.barrett || max_q < (std::uint64_t{1} << (bits - 2)),
                   "Barrett arithmetic needs every modulus below 2^" + std::to_string(bits - 2));
-        arith = c.barrett ? kBarrett : lazy ? kLazy : kStrict;
+        // Moduli that leave four spare bits (and whose reciprocal fits 32) take
+        // the headroom form of the lazy butterflies.
+        const bool headroom = lazy && bits == 64 && max_q < (std::uint64_t{1} << 60) && min_q >= (std::uint64_t{1} << 33);
+        arith = c.barrett ? kBarrett : headroom ? kHeadroom : lazy ? kLazy : kStrict;
         const std::uint64_t polys = c.polynomials.empty() ? c.batch : c.polynomials.size();
         require(polys >= 1 && polys <= 0xffffffffull, "NTT batch must be in [1, 2^32)");
         const bool offsets = !c.polynomials.empty();
@@ -161,10 +171,13 @@ struct EngineImplT {
         // (forward: natural in / bit-reversed out; inverse: the opposite).
         const bool perm_in = ct ? c.input_bit_reversed : !c.input_bit_reversed;
         const bool perm_out = ct ? !c.output_bit_reversed : c.output_bit_reversed;
-        if (log_n <= 12) {
+        if (log_n <= 12 || c.resident) {
             // One pass: whole polynomials per workgroup (one per tile if
-            // domains mix or polynomials sit at explicit offsets).
-            const int li = LB - int(log_n);
+            // domains mix or polynomials sit at explicit offsets, and from
+            // 2^12 points).
+            supported(log_n <= 12 || ntt_resident_offered(c.word_bits, log_n, polys, c.barrett),
+                      "one-pass NTT kernels end at 2^14 points");
+            const int li = std::max(LB - int(log_n), 0);
             supported((!mixed && !offsets) || li == 0, "mixed-domain or offset batches need log n >= 12");
             l1 = 0;
             l2 = log_n;
@@ -181,7 +194,7 @@ struct EngineImplT {
             L.prefix_bits = 0;
             L.last = true;
             launches.push_back(L);
-            json_shape = "{\"passes\":1,\"tile_log\":" + std::to_string(LB) + "}";
+            json_shape = "{\"passes\":1,\"tile_log\":" + std::to_string(std::max(LB, int(log_n))) + "}";
         } else {
             supported(log_n <= 20, "NTT lengths above 2^20 are not yet lowered for gfx950");
             l1 = std::uint32_t(split_l1(int(log_n)));
@@ -287,7 +300,7 @@ struct EngineImplT {
                     table[k] = pairs[k].w;
                 } else {
                     table[k] = pairs[k];
-                    if (ct && lazy) table[k].w = W(0) - table[k].w;  // lazy Cooley-Tukey butterflies take -w
+                    if (ct && arith == kLazy) table[k].w = W(0) - table[k].w;  // lazy Cooley-Tukey butterflies take -w
                 }
             }
             dd.tw = all_tables.size();
@@ -390,6 +403,32 @@ std::vector<std::uint32_t> ntt_other_splits(std::uint32_t log_n) {
     return out;
 }
 
+// Whole 2^13- / 2^14-point polynomials in one workgroup each: one round trip
+// through memory and one launch in place of two, but a batch has to fill the
+// chip. Measured with both lowerings over 5 .. 1024 polynomials, back-to-back
+// calls (two passes / resident, us, forward in native order):
+//   u32 2^13: 8 8.1 / 6.1, 64 8.1 / 6.3, 512 15.2 / 12.0, 1024 26.9 / 19.5
+//   u32 2^14: 64 8.1 / 9.9, 128 10.9 / 10.8, 192 13.5 / 11.8, 1024 57.7 / 45.3
+//   u64 2^13: 64 11.5 / 12.6, 128 13.5 / 13.4, 256 17.8 / 15.8, 1024 71 / 50
+//   u64 2^14: 64 15.5 / 22.5, 192 26.4 / 25.8, 256 36.4 / 27.8, 257 37.5 / 45.1,
+//             512 75 / 59
+// The other direction and orders cross at the same counts. A request is
+// offered the lowering (MEASURE, RNS Prepare) from about half of where it starts
+// to win; 2^13-point u32 rows from one per XCD.
+bool ntt_resident_offered(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys, bool barrett) {
+    if (barrett || (log_n != 13 && log_n != 14)) return false;
+    return polys >= (word_bits == 64 ? 96u : log_n == 14 ? 64u : 8u);
+}
+
+bool ntt_resident_default(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys) {
+    if (!ntt_resident_offered(word_bits, log_n, polys, false)) return false;
+    const std::uint64_t cus = std::uint64_t(device_cu_count());
+    // u64 2^14-point rows take a CU's LDS each and run in rounds of one per CU:
+    // where the last round is not nearly full the two passes are faster.
+    if (word_bits == 64 && log_n == 14) return polys * 5 >= (polys + cus - 1) / cus * cus * 4;
+    return (word_bits == 32 && log_n == 13) || polys > cus / 2;
+}
+
 std::size_t NttEngine::workspace_bytes() const {
     return impl_->u32 ? impl_->u32->workspace_bytes() : impl_->u64->workspace_bytes();
 }
@@ -421,11 +460,20 @@ bool wide_columns_default(const Request& r) { return r.word_bits == 32 && r.log_
 
 std::vector<std::uint32_t> other_splits(const Request& r) { return ntt_other_splits(r.log_n); }
 
-// Name of the static model's lowering: resident up to 2^12, then two passes.
-std::string default_name(const Request& r) {
-    return "ntt-u" + std::to_string(r.word_bits) + (r.negacyclic ? "-negacyclic" : "-cyclic") +
-           (r.log_n <= 12 ? "-resident-r16" : "-two-pass-r16");
+bool resident_default(const Request& r) { return ntt_resident_default(r.word_bits, r.log_n, r.batch); }
+
+std::string family_name(const Request& r) {
+    return "ntt-u" + std::to_string(r.word_bits) + (r.negacyclic ? "-negacyclic" : "-cyclic");
 }
+
+// Name of the lowerings that other options ride on: resident up to 2^12,
+// then two passes.
+std::string default_name(const Request& r) {
+    return family_name(r) + (r.log_n <= 12 ? "-resident-r16" : "-two-pass-r16");
+}
+
+// Whole 2^13- or 2^14-point polynomials, where they are a lowering of the request.
+std::string resident_name(const Request& r) { return family_name(r) + "-resident-r16"; }
 
 class NttExecutor final : public Executor {
   public:
@@ -467,6 +515,8 @@ class NttExecutor final : public Executor {
         c.force_strict = r.variant == default_name(r) + "-strict" + suffix;
         c.barrett = r.variant == default_name(r) + "-barrett" + suffix;
         c.wide_columns = r.variant.empty() ? wide_columns_default(r) : r.variant == default_name(r) + "-c32" + suffix;
+        if (r.log_n > 12)
+            c.resident = r.variant.empty() ? resident_default(r) : r.variant == resident_name(r) + suffix;
         for (const std::uint32_t h : other_splits(r))
             if (r.variant == default_name(r) + "-h" + std::to_string(h) + suffix) c.split_high = h;
         engine_ = std::make_unique<NttEngine>(c);
@@ -506,6 +556,8 @@ std::vector<std::string> ntt_candidates(const Request& r) {
     }
     for (const std::uint32_t h : other_splits(r)) names.push_back(default_name(r) + "-h" + std::to_string(h) + suffix);
     if (r.modulus < (std::uint64_t{1} << (r.word_bits - 2))) names.push_back(default_name(r) + "-barrett" + suffix);
+    if (ntt_resident_offered(r.word_bits, r.log_n, r.batch, false))
+        names.insert(resident_default(r) ? names.begin() : names.end(), resident_name(r) + suffix);
     return names;
 }
 

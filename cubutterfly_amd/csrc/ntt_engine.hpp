@@ -11,8 +11,8 @@
 // times n^-1. Natural/bit-reversed boundaries are LDS-staged permutations of
 // the first or last pass.
 //
-// Lengths up to 2^12 run in one pass (whole polynomials resident in a
-// workgroup); up to 2^24 in two passes over the high and low index bits,
+// Lengths up to 2^12 (2^13 and 2^14 in batches that fill the chip) run in one
+// pass (whole polynomials resident in a workgroup); others in two passes over the high and low index bits,
 // each an in-register radix-16 / LDS-exchange core, with the intermediate in
 // a workspace of polys * n words.
 #pragma once
@@ -46,6 +46,7 @@ struct NttEngineConfig {
     bool force_strict = false; // fully reduced butterflies even where lazy ones fit
     bool barrett = false;      // Barrett products on canonical values (moduli below 2^(word bits - 2))
     bool wide_columns = false; // two-pass: 32-column tiles in the column pass (`-c32`)
+    bool resident = false;     // 2^13 / 2^14 points: whole polynomials in one pass (ntt_resident_offered)
     std::uint32_t split_high = 0;  // two-pass: high (column-pass) bits; 0 = the planner's split (`-h<l1>`)
     std::vector<NttDomain> domains;
     std::vector<NttPolynomial> polynomials;  // empty: `batch` dense rows of domain 0
@@ -74,5 +75,11 @@ class NttEngine {
 // Two-pass high-bit splits other than the planner's that have kernels at
 // 2^log_n (the `-h<l1>` lowerings), empty elsewhere.
 std::vector<std::uint32_t> ntt_other_splits(std::uint32_t log_n);
+
+// Whether 2^log_n-point polynomials may run whole in one workgroup each
+// (NttEngineConfig::resident) where `polys` of them run at once.
+bool ntt_resident_offered(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys, bool barrett);
+// Whether that is the static model's choice.
+bool ntt_resident_default(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys);
 
 }  // namespace cbw

@@ -47,10 +47,11 @@ struct alignas(2 * sizeof(W)) TwPair {
 };
 
 // Arithmetic of a pass: Shoup products on fully reduced values ([0, 2q)
-// between stages), Shoup products on lazy ranges, or Barrett products on
+// between stages), Shoup products on lazy ranges, Barrett products on
 // canonical values with one constant per domain instead of a Shoup factor per
-// twiddle (tables of single words).
-constexpr int kStrict = 0, kLazy = 1, kBarrett = 2;
+// twiddle (tables of single words), or (u64, 2^33 <= q < 2^60) Shoup products
+// on ranges up to 16q, reduced once per phase (kHeadroom, see shoup_add).
+constexpr int kStrict = 0, kLazy = 1, kBarrett = 2, kHeadroom = 3;
 
 // A twiddle table entry: a Shoup pair, or the bare twiddle for Barrett.
 template <class W, int AR>
@@ -82,7 +83,7 @@ struct PassArgs {
     const std::uint64_t* out_off;
     std::uint32_t polys, tiles;
     std::uint32_t reduce_input;
-    std::uint32_t phase_off[3];  // chunk array of each phase, entries from the domain's table start
+    std::uint32_t phase_off[4];  // chunk array of each phase, entries from the domain's table start
     std::uint32_t tw_bytes;      // bytes of one domain's chunk tables (buffer range of the twiddle reads)
 };
 
@@ -92,20 +93,27 @@ struct PassArgs {
 // Cooley-Tukey (CT) walks the bits high -> low, windows [LT-4(P+1), LT-4P)
 // clamped at 0; Gentleman-Sande (GS) walks low -> high, windows [4P, 4P+4)
 // clamped at LT-4. A clamped window re-covers bits of its neighbour; only the
-// bits not yet done ("active" stages) are butterflied there.
+// bits not yet done ("active" stages) are butterflied there. Whole rows of
+// 2^13 and 2^14 points (kLongRow) take the CT windows in reverse order for GS
+// as well, so the clamped window is the lowest one in both directions and all
+// exchanges but one stay inside a wave (Pass::wave_local).
 
 constexpr int num_phases(int lt) { return (lt + kLE - 1) / kLE; }
 constexpr int imin(int a, int b) { return a < b ? a : b; }
 constexpr int imax(int a, int b) { return a > b ? a : b; }
 
+constexpr int kLongRow = 13;  // one-pass rows from 2^13 points
 constexpr int window_start(int lt, bool ct, int p) {
+    if (!ct && lt >= kLongRow) return window_start(lt, true, num_phases(lt) - 1 - p);
     return ct ? imax(lt - kLE * (p + 1), 0) : (kLE * p < lt - kLE ? kLE * p : imax(lt - kLE, 0));
 }
 constexpr int stage_hi(int lt, bool ct, int p) {
+    if (!ct && lt >= kLongRow) return stage_hi(lt, true, num_phases(lt) - 1 - p);
     const int ws = window_start(lt, ct, p);
     return ct ? imin(imin(ws + 3, lt - 1), lt - kLE * p - 1) : imin(ws + 3, lt - 1);
 }
 constexpr int stage_lo(int lt, bool ct, int p) {
+    if (!ct && lt >= kLongRow) return stage_lo(lt, true, num_phases(lt) - 1 - p);
     const int ws = window_start(lt, ct, p);
     return ct ? ws : imax(ws, kLE * p);
 }
@@ -149,7 +157,7 @@ constexpr std::uint64_t chunk_count(int lt, int prefix_bits, bool ct, int p) {
 // one-pass tiles, l1 for row tiles (their block index carries 2^l1 + row).
 template <class E>
 void append_pass_chunks(std::vector<E>& out, std::size_t base, const std::vector<E>& table, int lt,
-                        int prefix_bits, bool ct, bool last, std::uint32_t (&phase_off)[3]) {
+                        int prefix_bits, bool ct, bool last, std::uint32_t (&phase_off)[4]) {
     constexpr std::size_t per16 = 16 / sizeof(E) > 0 ? 16 / sizeof(E) : 1;
     for (int p = 0; p < num_phases(lt); ++p) {
         phase_off[p] = static_cast<std::uint32_t>(out.size() - base);
@@ -258,6 +266,95 @@ __device__ __forceinline__ void gs_scale_butterfly(W& x, W& y, const DeviceDomai
     y = shoup(u - v + span, d.last.w, d.last.wp, d.nq);
 }
 
+// ---- u64 arithmetic with headroom (q < 2^60, so 16q < 2^64) -------------------
+//
+// A 64-bit lazy butterfly is bound by VALU issue (about 4.5 cycles per wave64
+// instruction, the 32 x 32 + 64-bit v_mad_u64_u32 included), so what counts is
+// the number of instructions: 25 with the ranges of [0, 4q), 17 here, the
+// reductions included (measured with a radix-16 phase loop: 112 -> 89 cycles
+// per butterfly and wave). Three things save them:
+//  - no conditional subtraction per butterfly: every stage lets a value grow by
+//    3q, and a phase of four stages ends below 16q; reduce_wide brings it below
+//    3q again, once per phase;
+//  - the quotient leaves out the low x low partial product (one too small at
+//    most, hence 3q) and takes the middle sum's carry from the multiply-add;
+//  - the product's low word accumulates onto the butterfly's other operand in
+//    the same multiply-adds, and the high word in multiply-adds whose upper half
+//    is not used.
+
+// a b + c as one multiply-add: the compiler would split it into a multiply and
+// an add where only the low word is used, and into two multiply-adds where `b`
+// is half of a wave-uniform 64-bit value (whose zero extension it no longer
+// sees). `b` in a vector or a scalar register.
+__device__ __forceinline__ std::uint64_t mad_vv(std::uint32_t a, std::uint32_t b, std::uint64_t c) {
+    std::uint64_t r, carry;
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(carry) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ std::uint64_t mad_vs(std::uint32_t a, std::uint32_t b, std::uint64_t c) {
+    std::uint64_t r, carry;
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(carry) : "v"(a), "s"(b), "v"(c));
+    return r;
+}
+// x with `add` added to its high word.
+__device__ __forceinline__ std::uint64_t add_high(std::uint64_t x, std::uint32_t add) {
+    std::uint32_t hi = std::uint32_t(x >> 32);
+    asm("v_add_u32 %0, %1, %2" : "=v"(hi) : "v"(hi), "v"(add));
+    return (std::uint64_t(hi) << 32) | std::uint32_t(x);
+}
+
+// x + v, v = a w - Q q in [0, 3q) for any word a: Q is floor(a wp / 2^64) or one
+// less (P = a wp; the sum without its low x low product lies within 1 of P /
+// 2^64), and floor(a wp / 2^64) q itself is within 2q below a w.
+__device__ __forceinline__ std::uint64_t shoup_add(std::uint64_t x, std::uint64_t a, TwPair<std::uint64_t> t,
+                                                   std::uint64_t nq) {
+    const auto lo = [](std::uint64_t v) { return std::uint32_t(v); };
+    const auto hi = [](std::uint64_t v) { return std::uint32_t(v >> 32); };
+    const std::uint64_t m0 = std::uint64_t(lo(a)) * hi(t.wp);
+    std::uint64_t m1, carry, unused;
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(m1), "=s"(carry) : "v"(hi(a)), "v"(lo(t.wp)), "v"(m0));
+    const std::uint64_t h = std::uint64_t(hi(a)) * hi(t.wp) + hi(m1);
+    // A vector instruction may read a scalar register that another wrote after
+    // two wait states, which the compiler does not count across asm blocks: the
+    // multiply-add of h, which needs m1 and is needed here, is one, the s_nop the
+    // other.
+    std::uint32_t qh = hi(h);
+    asm("s_nop 0\n\tv_addc_co_u32_e64 %0, %1, %2, 0, %3" : "=v"(qh), "=s"(unused) : "v"(qh), "s"(carry));
+    const std::uint64_t p = mad_vs(lo(h), lo(nq), std::uint64_t(lo(a)) * lo(t.w) + x);
+    std::uint64_t k = std::uint64_t(lo(a)) * hi(t.w);
+    k = mad_vv(hi(a), lo(t.w), k);
+    k = mad_vs(lo(h), hi(nq), k);
+    k = mad_vs(qh, lo(nq), k);
+    return add_high(p, lo(k));
+}
+
+// Any word to [0, 3q): k = floor(x.hi m / 2^32), m = floor(2^64 / q) (the Shoup
+// factor of 1), is at most x / q and above x / q - 2^32 / q - 1 - 1.
+__device__ __forceinline__ std::uint64_t reduce_wide(std::uint64_t x, const DeviceDomain<std::uint64_t>& d) {
+    const std::uint32_t k = __umulhi(std::uint32_t(x >> 32), std::uint32_t(d.rwp));
+    const std::uint64_t p = mad_vs(k, std::uint32_t(d.nq), x);
+    return add_high(p, k * std::uint32_t(d.nq >> 32));
+}
+
+// Ranges of the headroom arithmetic, in units of q. Forward: a stage adds 3 to
+// every value; a phase that would pass 16 reduces its values to 3 first.
+// Inverse: sums double, products are 3; see Pass::headroom_stages.
+constexpr int kGrowth = 3, kHeadroomLimit = 16, kReduced = 3;
+constexpr int forward_bound_before(int lt, int p, int bound);
+// Bound after phase p of a forward pass whose values enter below `bound`.
+constexpr int forward_bound_after(int lt, int p, int bound) {
+    const int b = p < 0 ? bound : forward_bound_before(lt, p, bound);
+    return p < 0 ? b : b + kGrowth * active_stages(lt, true, p);
+}
+// Bound entering phase p, after the reduction where it needs one.
+constexpr int forward_bound_before(int lt, int p, int bound) {
+    const int b = forward_bound_after(lt, p - 1, bound);
+    return b + kGrowth * active_stages(lt, true, p) > kHeadroomLimit ? kReduced : b;
+}
+constexpr bool forward_reduces(int lt, int p, int bound) {
+    return forward_bound_after(lt, p - 1, bound) + kGrowth * active_stages(lt, true, p) > kHeadroomLimit;
+}
+
 // Barrett (the constants of the reference's GPU-NTT-compatible provider,
 // src/ntt_hybrid2d.cuh:53-71, mu = floor(2^(2b+1) / q) for the bit length b
 // of q, q < 2^(k-2)): for canonical a, w < q, P = a w < 2^(2b),
@@ -331,7 +428,14 @@ __device__ __forceinline__ std::uint32_t phase_index(std::uint32_t t, std::uint3
 // over the row bits and index bit 7), where the single pitch of 273 words
 // (17 modulo 32) put two lanes on each bank (4 conflict cycles per ds_*2_b32
 // instruction, measured, and reproduced by enumerating the accesses).
-template <bool COL, bool SWZ, int LT, int LI, bool BANKED = false>
+//
+// Whole rows of 2^13 and 2^14 points (LONG: the word bytes, 0 elsewhere) add
+// a second pad, one word for each step of the top index bits (u64: the top
+// four, u32: those from bit 9): a bit-reversed staging walks a wave's lanes
+// over the top bits, which the 1-in-16 pad alone puts on one bank. The image
+// stays a sum over index bits. Conflict-free for the exchanges and the
+// staging by enumeration (u32 2^13: two lanes of each bank in the staging).
+template <bool COL, bool SWZ, int LT, int LI, bool BANKED = false, int LONG = 0>
 struct Lds {
     static_assert(!BANKED || (!COL && LT == 8 && LI <= 5), "banked row offsets cover 2^8-point rows, up to 32");
     // Row bit j > 0 contributes 545 * 2^(j - 1): the bits above bit 0 are
@@ -342,12 +446,19 @@ struct Lds {
     // Without the swizzle, addr() is a sum of terms over disjoint index bit
     // fields, so addr(a | b) = addr(a) + addr(b) for disjoint a, b.
     static constexpr bool kLinear = !(COL && SWZ);
+    static_assert(LONG == 0 || (!COL && !BANKED && LI == 0 && (LT == 13 || LT == 14)), "whole long rows");
+    static __host__ __device__ constexpr std::uint32_t long_row(std::uint32_t x) {
+        return x + (x >> 4) + (LONG == 8 ? x >> (LT - 4) : (x >> 9) << (14 - LT));
+    }
     static constexpr std::uint32_t kWords =
-        COL      ? (1u << LT) * ((1u << LI) + 1u)
+        LONG     ? long_row((1u << LT) - 1u) + 1u
+        : COL    ? (1u << LT) * ((1u << LI) + 1u)
         : BANKED ? row_offset((1u << LI) - 1u) + (1u << LT) + (1u << LT >> 4) - 1u
                  : (1u << LI) * ((1u << LT) + (1u << LT >> 4) + 1u);
     static __device__ __forceinline__ std::uint32_t addr(std::uint32_t i) {
-        if constexpr (COL) {
+        if constexpr (LONG != 0) {
+            return long_row(i);
+        } else if constexpr (COL) {
             const std::uint32_t cc = i & ((1u << LI) - 1u), x = i >> LI;
             if constexpr (SWZ) {
                 constexpr int top = LT > LI ? LT - LI : 0;
@@ -382,6 +493,8 @@ template <class W, int AR, int LT, int LI, bool COL, bool CT, bool PIN, bool POU
 struct Pass {
     static constexpr bool LAZY = AR == kLazy;
     static constexpr bool BARRETT = AR == kBarrett;
+    static constexpr bool HEADROOM = AR == kHeadroom;
+    static_assert(!HEADROOM || sizeof(W) == 8, "headroom arithmetic is for 64-bit words");
     using E = Entry<W, AR>;
     static constexpr int LB = LT + LI;
     static constexpr std::uint32_t T = 1u << (LB - kLE);
@@ -392,7 +505,8 @@ struct Pass {
     // Rows of a permuted two-pass ROW tile are bitrev(k0 + rr).
     static constexpr bool kPermRows = !COL && !SINGLE && (PIN || POUT);
     static constexpr std::uint32_t kPolyBytes = std::uint32_t(sizeof(W)) << kLogN;
-    using L = Lds<COL, COL && (PIN || POUT), LT, LI, !COL && sizeof(W) == 4 && LT == 8 && LI <= 5>;
+    using L = Lds<COL, COL && (PIN || POUT), LT, LI, !COL && sizeof(W) == 4 && LT == 8 && LI <= 5,
+                  SINGLE && LT >= kLongRow ? int(sizeof(W)) : 0>;
     // Stores of two-pass inverse (Gentleman-Sande) tiles write through the L2
     // (sc0 sc1), so the end-of-kernel write-back has little left to flush;
     // measured 5-6% faster per C2 / C4 step. Forward passes keep write-back
@@ -409,21 +523,22 @@ struct Pass {
     static constexpr int kStoreAux = (!CT && !SINGLE) || (CT && !SINGLE && !COL && POUT) ? 17
                                      : (COL && CT && !SINGLE && (sizeof(W) << LI) >= 128) ? 2
                                                                                           : 0;
-    // Row tiles of at most 2^10-point rows: every phase layout keeps a row in
-    // 2^(LT-4) <= 64 consecutive threads (phase_index puts the row bits at
-    // t >> (LT - 4)), so the register-window exchanges never leave a wave.
-    // Their barriers would only hold the workgroup's waves in step; a wave
-    // that has its data computes while the others still wait for theirs.
+    // A register window starting at tile bit S <= 6 leaves tile bits 10 and up
+    // to the wave index (phase_index: thread bits from 6 up are tile bits from
+    // 10 up), so an exchange between two such windows never leaves a wave: all
+    // exchanges of row tiles of at most 2^10-point rows, and all but one of
+    // longer rows. A barrier would only hold the workgroup's waves in step; a
+    // wave that has its data computes while the others still wait for theirs.
     // The staged boundary permutations (PIN / POUT) mix rows across waves
     // and keep their barriers.
-    static constexpr bool kWaveLocal = !COL && LT - kLE <= 6;
+    static constexpr bool wave_local(int from, int to) { return !COL && from <= 6 && to <= 6; }
     // Forward row tiles whose output stays in the transform's native order
     // end with every thread holding 16 consecutive outputs of one row, so a
     // store instruction would put its 64 lanes 16 words apart (64 cache lines
     // per instruction). A wave's 1024 outputs are one contiguous run, and
     // they go through the wave's own LDS rows instead: each 16-byte store
     // instruction then covers 64 x 16 contiguous bytes.
-    static constexpr bool kStagedStore = !COL && CT && kLast && !POUT && kWaveLocal && LT + LI >= 10;
+    static constexpr bool kStagedStore = !COL && CT && kLast && !POUT && LT + LI >= 10;
     static constexpr int kStagedAux = SINGLE ? 0 : 17;
     // (The mirror image, the first inverse pass loading its native-order rows
     // as contiguous runs and moving them into the phase-0 layout through the
@@ -441,7 +556,7 @@ struct Pass {
     }
     static constexpr std::uint32_t run_offset(int k) { return 64u * std::uint32_t(kPer) * std::uint32_t(k); }
     static_assert(SINGLE ? (L1 == 0 && L2 == LT) : (COL ? LT == L1 : LT == L2), "pass bits");
-    static_assert(LT >= 1 && LB >= kLE && LB <= 13, "tile shape");
+    static_assert(LT >= 1 && LB >= kLE && LB <= 14, "tile shape");
 
     template <int P>
     static constexpr int tile_window() {
@@ -621,6 +736,10 @@ struct Pass {
 
     template <int P>
     static __device__ __forceinline__ void stages(W (&v)[kE], const Chunk<P>& c, const DeviceDomain<W>& d) {
+        if constexpr (HEADROOM) {
+            headroom_stages<P>(v, c, d);
+            return;
+        }
         constexpr int ws = window_start(LT, CT, P);
 #pragma unroll
         for (int s = 0; s < active_stages(LT, CT, P); ++s) {
@@ -669,6 +788,77 @@ struct Pass {
         }
     }
 
+    // Bound (in units of q) of the values entering the first pass and, for the
+    // second pass of a forward transform, what the column pass left.
+    static constexpr int kEntry = 4;
+    static constexpr int kForwardEntry =
+        SINGLE || COL ? kEntry : forward_bound_after(L1, num_phases(L1) - 1, kEntry);
+    static constexpr int kForwardExit = forward_bound_after(LT, kPhases - 1, kForwardEntry);
+
+    // The phase's butterflies in headroom arithmetic. `bound[r]` is v[r]'s range
+    // in units of q: the loops unroll completely, so it is known at compile time
+    // and only the reductions it asks for remain.
+    template <int P>
+    static __device__ __forceinline__ void headroom_stages(W (&v)[kE], const Chunk<P>& c, const DeviceDomain<W>& d) {
+        constexpr int ws = window_start(LT, CT, P);
+        if constexpr (CT && forward_reduces(LT, P, kForwardEntry)) {
+#pragma unroll
+            for (int r = 0; r < kE; ++r) v[r] = reduce_wide(v[r], d);
+        }
+        // Multiples of q that keep differences positive, in scalar registers
+        // (opaque: the compiler would multiply per butterfly).
+        W q3 = 3 * d.q, q6 = 6 * d.q, q12 = 12 * d.q;
+        asm("" : "+s"(q3), "+s"(q6), "+s"(q12));
+        int bound[kE];
+#pragma unroll
+        for (int r = 0; r < kE; ++r) bound[r] = kReduced;
+#pragma unroll
+        for (int s = 0; s < active_stages(LT, CT, P); ++s) {
+            const int k = exec_stage(LT, CT, P, s);
+            const int jb = k - ws;
+            const std::uint32_t gmask = (1u << (LT - 1 - k)) - 1u;
+            const bool scale = scale_stage(LT, CT, kLast, k);
+            const int off = chunk_offset(LT, CT, kLast, P, s);
+#pragma unroll
+            for (int g = 0; g < (1 << (kLE - 1 - jb)); ++g) {
+                const int e = scale ? 0 : off + int(std::uint32_t(g) & gmask);
+                const TwPair<W> tp{(W(c.raw[e][1]) << 32) | c.raw[e][0], (W(c.raw[e][3]) << 32) | c.raw[e][2]};
+#pragma unroll
+                for (int lo = 0; lo < (1 << jb); ++lo) {
+                    const int r = (g << (jb + 1)) | lo;
+                    const int r2 = r | (1 << jb);
+                    if constexpr (CT) {
+                        // x + v and x + 3q - v = 2x + 3q - (x + v). (The empty
+                        // asm keeps 2x + 3q one shift-add.)
+                        W twice = (v[r] << 1) + q3;
+                        asm("" : "+v"(twice));
+                        v[r] = shoup_add(v[r], v[r2], tp, d.nq);
+                        v[r2] = twice - v[r];
+                    } else {
+                        // Both sides of a pair have the same bound: 3, 6 or 12.
+                        if (bound[r] + bound[r2] > kHeadroomLimit) {
+                            v[r] = reduce_wide(v[r], d);
+                            v[r2] = reduce_wide(v[r2], d);
+                            bound[r] = bound[r2] = kReduced;
+                        }
+                        const W sum = v[r] + v[r2];
+                        const W span = bound[r2] <= 3 ? q3 : bound[r2] <= 6 ? q6 : q12;
+                        const W diff = v[r] + span - v[r2];
+                        v[r] = scale ? shoup_add(0, sum, d.ninv, d.nq) : sum;
+                        v[r2] = shoup_add(0, diff, scale ? d.last : tp, d.nq);
+                        bound[r] = scale ? kReduced : bound[r] + bound[r2];
+                        bound[r2] = kReduced;
+                    }
+                }
+            }
+        }
+        if constexpr (!CT) {  // every phase and pass of the inverse starts from kReduced
+#pragma unroll
+            for (int r = 0; r < kE; ++r)
+                if (bound[r] > kReduced) v[r] = reduce_wide(v[r], d);
+        }
+    }
+
     // Register window FROM -> TO through the LDS image. `between` runs
     // between the writes and the second barrier: the next phase's twiddle
     // loads go there, so their latency overlaps the barrier wait and their
@@ -676,12 +866,12 @@ struct Pass {
     // phase's chunk up front kept them all live and cost occupancy).
     template <int FROM, int TO, class Between>
     static __device__ __forceinline__ void exchange(W (&v)[kE], W* lds, std::uint32_t t, Between&& between) {
-        if constexpr (kWaveLocal) wave_lds_fence();
+        if constexpr (wave_local(FROM, TO)) wave_lds_fence();
         else lds_barrier();
 #pragma unroll
         for (int r = 0; r < kE; ++r) lds[L::template at<FROM>(t, r)] = v[r];
         between();
-        if constexpr (kWaveLocal) wave_lds_fence();
+        if constexpr (wave_local(FROM, TO)) wave_lds_fence();
         else lds_barrier();
 #pragma unroll
         for (int r = 0; r < kE; ++r) v[r] = lds[L::template at<TO>(t, r)];
@@ -720,15 +910,21 @@ struct Pass {
             for (int r = 0; r < kE; ++r) v[r] = lds[L::template at<tile_window<0>()>(t, r)];
         }
         if (kFirst && a.reduce_input) {
-            // Arbitrary input words -> [0, 2q). A Cooley-Tukey first stage
+            // Arbitrary input words -> [0, 2q) ([0, 3q) with headroom). A Cooley-Tukey first stage
             // multiplies its upper operands by Shoup twiddles (any word is
             // fine there), so only the lower half needs it. Barrett products
             // need canonical operands: every word is reduced to [0, q).
             constexpr int top = CT ? stage_hi(LT, CT, 0) - window_start(LT, CT, 0) : kLE;
 #pragma unroll
             for (int r = 0; r < kE; ++r) {
-                if constexpr (BARRETT) v[r] = reduce_once(shoup(v[r], W(1), d.rwp, d.nq), d.q);
-                else if (!CT || LT < kLE || !((r >> top) & 1)) v[r] = shoup(v[r], W(1), d.rwp, d.nq);
+                const bool needed = !CT || LT < kLE || !((r >> top) & 1);
+                if constexpr (BARRETT) {
+                    v[r] = reduce_once(shoup(v[r], W(1), d.rwp, d.nq), d.q);
+                } else if constexpr (HEADROOM) {
+                    if (needed) v[r] = reduce_wide(v[r], d);
+                } else {
+                    if (needed) v[r] = shoup(v[r], W(1), d.rwp, d.nq);
+                }
             }
         }
         stages<0>(v, c0, d);
@@ -744,12 +940,19 @@ struct Pass {
                                                          [&] { load_chunk<2>(c2, a, tl, t, twiddles(a, d)); });
             stages<2>(v, c2, d);
         }
+        if constexpr (kPhases > 3) {
+            Chunk<3> c3;
+            exchange<tile_window<2>(), tile_window<3>()>(v, lds, t,
+                                                         [&] { load_chunk<3>(c3, a, tl, t, twiddles(a, d)); });
+            stages<3>(v, c3, d);
+        }
         constexpr int wl = tile_window<kPhases - 1>();
         if constexpr (kLast) {
 #pragma unroll
             for (int r = 0; r < kE; ++r) {
                 W x = v[r];
-                if constexpr (CT && LAZY) x = csub(x, d.q2);
+                if constexpr (HEADROOM && CT && kForwardExit > 4) x = reduce_wide(x, d);
+                if constexpr ((CT && LAZY) || HEADROOM) x = csub(x, d.q2);
                 v[r] = csub(x, d.q);
             }
         }
@@ -895,6 +1098,14 @@ constexpr int kColLines = 4;
 constexpr int kWideColLines = 5;
 constexpr int row_lines(int l1, int l2) { return l1 < kTileLog - l2 ? l1 : kTileLog - l2; }
 
+// Whole polynomials of 2^13 and 2^14 points in one pass: one per workgroup of
+// 512 or 1024 threads.
+template <class W, int AR>
+void add_long_rows() {
+    add_single<W, AR, 13, 13>();
+    add_single<W, AR, 14, 14>();
+}
+
 // Column passes of one split with 32-column tiles, where they fit.
 template <class W, int AR, int L1, int L2>
 void add_wide_columns() {
@@ -937,6 +1148,28 @@ void add_split() {
     add_rows<W, AR, L1, LOG_N - L1>();
 }
 
+// u64 pass shapes beyond the planner's static choice: the neighbouring splits of
+// 2^15..2^17 (16- and 32-column tiles) and 32-column tiles at the planner's
+// split of every two-pass length. They are candidates of MEASURE and RNS Prepare.
+template <int AR>
+void add_alt_u64() {
+    using W = std::uint64_t;
+    add_split<W, AR, 15, 6>();
+    add_split<W, AR, 15, 8>();
+    add_split<W, AR, 16, 7>();
+    add_split<W, AR, 16, 9>();
+    add_split<W, AR, 17, 7>();
+    add_split<W, AR, 17, 9>();
+    add_wide_columns<W, AR, 6, 7>();
+    add_wide_columns<W, AR, 7, 7>();
+    add_wide_columns<W, AR, 7, 8>();
+    add_wide_columns<W, AR, 8, 8>();
+    add_wide_columns<W, AR, 8, 9>();
+    add_wide_columns<W, AR, 8, 10>();
+    add_wide_columns<W, AR, 8, 11>();
+    add_wide_columns<W, AR, 8, 12>();
+}
+
 // 4 KiWord tiles; columns of 64 B (u32) / 128 B (u64).
 template <class W, int AR>
 void register_all() {
@@ -969,8 +1202,12 @@ void register_u64_lazy();
 void register_u64_strict();
 void register_u32_barrett();
 void register_u64_barrett();
+void register_u64_headroom();
 void register_alt_u32();
 void register_alt_u64();
+void register_alt_u64_headroom();
+void register_long_rows_u32();
+void register_long_rows_u64();
 
 // Splits l1 of two-pass lengths with kernels: the planner's split_l1 and the
 // neighbouring ones that ntt_alt_u32.hip and ntt_alt_u64.hip instantiate.

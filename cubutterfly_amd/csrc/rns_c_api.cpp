@@ -196,9 +196,7 @@ struct RnsMapping {
     bool wide = false;        // 32-column tiles in the column pass
     std::uint32_t split = 0;  // high (column-pass) bits; 0 = the planner's split
     bool barrett = false;     // Barrett products (one constant per domain, single-word twiddle tables)
-    bool operator==(const RnsMapping& o) const {
-        return strict == o.strict && wide == o.wide && split == o.split && barrett == o.barrett;
-    }
+    bool resident = false;    // 2^13 / 2^14 points: whole polynomials in one pass
 };
 
 // A lowering's engines: the transform, and for one-pass in-place plans whose
@@ -223,6 +221,7 @@ RnsLowering lower(const RnsConfig& config, const RnsMapping& m, bool same_offset
     e.barrett = m.barrett;
     e.wide_columns = m.wide;
     e.split_high = m.split;
+    e.resident = m.resident;
     e.domains = config.domains;
     e.polynomials = config.polynomials;
     RnsLowering l;
@@ -230,7 +229,7 @@ RnsLowering lower(const RnsConfig& config, const RnsMapping& m, bool same_offset
     l.engine = std::make_unique<cbw::NttEngine>(e);
     const std::uint64_t n = std::uint64_t{1} << config.log_n;
     l.scratch_bytes = l.engine->workspace_bytes();
-    if (l.engine->passes() == 1 && !same_offsets) {
+    if (l.engine->passes() == 1 && !same_offsets && !m.resident) {
         auto dense = e;
         for (std::size_t p = 0; p < dense.polynomials.size(); ++p) dense.polynomials[p].output_offset = p * n;
         l.to_scratch = std::make_unique<cbw::NttEngine>(dense);
@@ -239,8 +238,10 @@ RnsLowering lower(const RnsConfig& config, const RnsMapping& m, bool same_offset
     return l;
 }
 
-// Mappings Prepare may choose for a request, the static plan first.
-std::vector<RnsMapping> candidates(const RnsConfig& c) {
+// Mappings Prepare may choose for a request, the static plan first. `moving`:
+// in place with some polynomial at another offset on the output side, which a
+// one-pass tile would write over words another tile has not read.
+std::vector<RnsMapping> candidates(const RnsConfig& c, bool moving) {
     std::uint64_t max_q = 0;
     for (const auto& d : c.domains) max_q = std::max(max_q, d.modulus);
     // Lazy butterflies need 4q below the word: where they fit they are the
@@ -254,6 +255,8 @@ std::vector<RnsMapping> candidates(const RnsConfig& c) {
         if (c.log_n <= 12) continue;  // one pass: no columns, no split
         out.push_back({strict, true, 0, false});
         for (const std::uint32_t split : cbw::ntt_other_splits(c.log_n)) out.push_back({strict, false, split, false});
+        if (!moving && cbw::ntt_resident_offered(64, c.log_n, c.polynomials.size(), false))
+            out.push_back({strict, false, 0, false, true});
     }
     // Barrett products, as the reference's mapping offers them beside Shoup
     // (src/rns_ntt.cu:331-346, rejected there too for moduli of 2^62 or more),
@@ -263,8 +266,8 @@ std::vector<RnsMapping> candidates(const RnsConfig& c) {
 }
 
 std::string mapping_name(const RnsMapping& m) {
-    return std::string(m.barrett ? "barrett" : m.strict ? "strict" : "lazy") + (m.wide ? "-c32" : "-c16") +
-           (m.split ? "-h" + std::to_string(m.split) : "");
+    return std::string(m.barrett ? "barrett" : m.strict ? "strict" : "lazy") +
+           (m.resident ? "-resident" : m.wide ? "-c32" : "-c16") + (m.split ? "-h" + std::to_string(m.split) : "");
 }
 
 struct RnsMeasurement {
@@ -436,7 +439,7 @@ RnsLowering sweep(cubutterflyRnsPlanOpaque& plan, bool in_place, unsigned repeti
     std::uint64_t* destination = in_place ? in.as<std::uint64_t>() : out.as<std::uint64_t>();
     cbw::hip_check(hipMemsetAsync(in.as<void>(), 0, in_words * 8, stream), "RNS prepare fill");
     std::vector<RnsLowering> lowerings;
-    for (const RnsMapping& m : candidates(plan.config)) {
+    for (const RnsMapping& m : candidates(plan.config, in_place && !plan.same_offsets)) {
         try {
             lowerings.push_back(lower(plan.config, m, plan.same_offsets));
         } catch (const cbw::NotSupported&) {
@@ -536,7 +539,7 @@ int cubutterflyRnsCreate(const char* config_json_text, cubutterflyRnsPlan* resul
                                          [](const cbw::NttPolynomial& p) { return p.input_offset == p.output_offset; });
         // The static plan until Prepare selects (private scratch allocated
         // here, outside execution; reference :286-366).
-        plan->select(lower(plan->config, candidates(plan->config).front(), plan->same_offsets));
+        plan->select(lower(plan->config, candidates(plan->config, false).front(), plan->same_offsets));
         *result = plan.release();
     });
 }
@@ -599,7 +602,7 @@ int cubutterflyRnsPrepare(cubutterflyRnsPlan plan, int placement, const char* ca
             // The record names one of this request's candidates; it is rebuilt,
             // never trusted beyond that.
             const std::string selected = record.at("selected").as_string("selected");
-            const auto options = candidates(plan->config);
+            const auto options = candidates(plan->config, placement == 1 && !plan->same_offsets);
             const auto it = std::find_if(options.begin(), options.end(),
                                          [&](const RnsMapping& m) { return mapping_name(m) == selected; });
             require(it != options.end(), "RNS cache record selects no mapping of this request: " + selected);
