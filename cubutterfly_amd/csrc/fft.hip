@@ -51,6 +51,8 @@ struct FftArgs {
     // Elements between consecutive transforms of the input / output buffer:
     // n when packed, a caller's row pitch otherwise (one transform per tile).
     std::uint64_t in_pitch, out_pitch;
+    // ORD bit 6 (ragged rows): elements present in a row of the ragged side.
+    std::uint32_t row_len;
 };
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
@@ -214,7 +216,12 @@ constexpr int pass_digit_bits(int lb, bool single, int ord) { return (ord & 16) 
 // output k = k1 + 2^l1 k2 belongs at bitrev(k) = bitrev(k1) 2^l2 +
 // bitrev(k2), and the row pass reads tile row k1 from row bitrev(k1) of the
 // intermediate, so each row goes back to the row it came from, in the DIF
-// result's own order (no reversal, no transpose).
+// result's own order (no reversal, no transpose). Bit 6 gives the input rows
+// (forward) or the output rows (inverse) of one-pass tiles row_len elements in
+// place of 2^LT, in_pitch / out_pitch apart: the forward reads zeros past a row's
+// end, the inverse drops what lies past it (the zero-extended embedding without
+// a padded copy). One-row tiles leave both to the buffer range check; tiles of
+// several rows send the lane offsets past a row's end out of the range.
 template <int LT, int LI, bool COL, bool SINGLE, bool INV, int ORD = 0>
 struct FftPass {
     static constexpr int LB = LT + LI;
@@ -227,6 +234,9 @@ struct FftPass {
     // and for the 4-bit one-pass tiles of 2^13 / 2^14 points, whose bases
     // beyond the third are fetched digit by digit.
     static constexpr bool kPrefetch = DB == 5 || kPhases <= 2 || (ORD & 16) != 0;
+    static constexpr bool kRaggedIn = (ORD & 64) != 0 && !INV;
+    static constexpr bool kRaggedOut = (ORD & 64) != 0 && INV;
+    static_assert((ORD & 64) == 0 || (SINGLE && ORD == 64), "ragged rows are one-pass rows in natural order");
     static constexpr bool kPairedColumns = COL && LI == 6 && kE == 16;
     using L = FftLds<COL, LT, LI, SINGLE, kPairedColumns, DB>;
 
@@ -364,7 +374,7 @@ struct FftPass {
     // The relabelled reads keep every 16-lane group on 16 distinct bank
     // pairs of the XOR image: its lanes vary position bits LT-5..LT-2, the
     // image's second key field.
-    static constexpr bool kDirectStore = SINGLE && LI == 0 && ORD == 0 && DB == 5;
+    static constexpr bool kDirectStore = SINGLE && LI == 0 && (ORD & ~64) == 0 && DB == 5;
     static __device__ __forceinline__ std::uint32_t last_thread_index(std::uint32_t t) {
         const std::uint32_t l = t & 63u, w = t >> 6;
         return ((l & 1u) << (LT - 2)) | (((l >> 1) & 1u) << (LT - 3)) | (((l >> 2) & 1u) << (LT - 4)) |
@@ -418,9 +428,22 @@ struct FftPass {
 
     // Bytes of the tile's span: a one-pass tile's existing rows (the range
     // check zero-fills loads and drops stores past them), else its transform.
-    static __device__ __forceinline__ std::uint32_t span_bytes(const FftArgs& a, const Tile& tl, std::uint32_t m) {
-        if constexpr (SINGLE) return min(1u << LI, a.rows - tl.row0) << (LT + 3);
+    // RAGGED: the rows' existing elements, up to the last row's last one.
+    template <bool RAGGED = false>
+    static __device__ __forceinline__ std::uint32_t span_bytes(const FftArgs& a, const Tile& tl, std::uint32_t m,
+                                                               std::uint64_t pitch = 0) {
+        if constexpr (RAGGED)
+            return 8u * ((min(1u << LI, a.rows - tl.row0) - 1u) * std::uint32_t(pitch) + a.row_len);
+        else if constexpr (SINGLE) return min(1u << LI, a.rows - tl.row0) << (LT + 3);
         else return 8u << m;
+    }
+    // Byte offset of tile element i on the ragged side, past every range where
+    // its row (or, in a partial last tile, the row itself) is absent.
+    static __device__ __forceinline__ std::uint32_t ragged_offset(const FftArgs& a, const Tile& tl, std::uint64_t pitch,
+                                                                  std::uint32_t i) {
+        const std::uint32_t x = i & ((1u << LT) - 1u), rr = i >> LT;
+        if constexpr (LI == 0) return x * 8u;  // the span ends with the row
+        else return x < a.row_len && rr < a.rows - tl.row0 ? (rr * std::uint32_t(pitch) + x) * 8u : 0xfffffff8u;
     }
 
     // Element offsets split into a per-thread part and a wave-uniform
@@ -498,7 +521,15 @@ struct FftPass {
                                                 float2 (&v)[kE], bool valid = true) {
         constexpr int w0 = tile_window<0>();
         const __amdgpu_buffer_rsrc_t src =
-            make_rsrc(a.in + span_base(a, tl, a.in_pitch), valid ? span_bytes(a, tl, m) : 0u);
+            make_rsrc(a.in + span_base(a, tl, a.in_pitch), valid ? span_bytes<kRaggedIn>(a, tl, m, a.in_pitch) : 0u);
+        if constexpr (kRaggedIn) {
+            const std::uint32_t it = index<w0>(t, 0);
+#pragma unroll
+            for (int r = R0; r < R1; ++r) {
+                v[r] = buffer_load<float2, kLoadAux>(src, ragged_offset(a, tl, a.in_pitch, it | index<w0>(0, r)));
+            }
+            return;
+        }
         if constexpr (kPairedColumns) {
             static_assert(R0 % 2 == 0 && R1 % 2 == 0, "register pairs");
             static_assert(w0 == LI + 4, "digit 0 holds the top four of eight row bits");
@@ -561,7 +592,7 @@ struct FftPass {
             at(integral_constant<int, 6>{});
         }
         constexpr int wl = tile_window<kPhases - 1>();
-        const __amdgpu_buffer_rsrc_t dst = make_rsrc(a.out + span_base(a, tl, a.out_pitch), span_bytes(a, tl, m));
+        const __amdgpu_buffer_rsrc_t dst = make_rsrc(a.out + span_base(a, tl, a.out_pitch), span_bytes<kRaggedOut>(a, tl, m, a.out_pitch));
         if constexpr (COL) {  // intermediate: same positions
             at(integral_constant<int, 2 * kPhases - 1>{});
             if constexpr (kPairedColumns) {
@@ -589,7 +620,12 @@ struct FftPass {
             static_assert(wl == 0, "registers hold tile positions 0-4");
             at(integral_constant<int, 2 * kPhases - 1>{});
             const std::uint32_t kt = brev(last_thread_index(t), LT) * 8u;
-            if (a.scale == 1.0f) {
+            if constexpr (kRaggedOut) {
+#pragma unroll
+                for (int r = 0; r < kE; ++r)
+                    buffer_store<float2, kStoreAux>(make_float2(v[r].x * a.scale, v[r].y * a.scale), dst,
+                                                    kt + brev_const(std::uint32_t(r), LT) * 8u);
+            } else if (a.scale == 1.0f) {
 #pragma unroll
                 for (int r = 0; r < kE; ++r) store_at(v[r], dst, kt, brev_const(std::uint32_t(r), LT) * 8u);
             } else {
@@ -612,6 +648,17 @@ struct FftPass {
         }
         std::uint32_t it, ot;
         staged(a, tl, t, it, ot);
+        if constexpr (kRaggedOut) {
+#pragma unroll
+            for (int r = 0; r < kE; ++r) {
+                std::uint32_t ir, orr;
+                staged(a, Tile{}, T * std::uint32_t(r), ir, orr);
+                const float2 x = lds[L::split(it, ir)];
+                buffer_store<float2, kStoreAux>(make_float2(x.x * a.scale, x.y * a.scale), dst,
+                                                ragged_offset(a, tl, a.out_pitch, ot + orr));
+            }
+            return;
+        }
         // Unnormalised plans (scale 1) skip the products: a wave-uniform
         // branch over two copies of the store loop.
         if (a.scale == 1.0f) {
@@ -639,7 +686,7 @@ struct FftPass {
     // (2t) and a register part (2 T r) over disjoint bits, and output 2j + 1
     // differs from it in one bit that is clear in both parts: the top one
     // after bit reversal, bit 0 otherwise.
-    static constexpr bool kPairedStore = SINGLE && LI == 0;
+    static constexpr bool kPairedStore = SINGLE && LI == 0 && !kRaggedOut;
     static __device__ __forceinline__ std::uint32_t pair_index(std::uint32_t g) {
         return (ORD & 2) != 0 ? g : brev(g, LT);
     }
@@ -916,6 +963,8 @@ void add() {
         registry()[Key{LT, LI, COL, SINGLE, true, 2}] = &launch<LT, LI, COL, SINGLE, true, 2>;
         registry()[Key{LT, LI, COL, SINGLE, false, 3}] = &launch<LT, LI, COL, SINGLE, false, 3>;
         registry()[Key{LT, LI, COL, SINGLE, true, 3}] = &launch<LT, LI, COL, SINGLE, true, 3>;
+        registry()[Key{LT, LI, COL, SINGLE, false, 64}] = &launch<LT, LI, COL, SINGLE, false, 64>;  // ragged rows
+        registry()[Key{LT, LI, COL, SINGLE, true, 64}] = &launch<LT, LI, COL, SINGLE, true, 64>;
     }
     if constexpr (!COL && !SINGLE) {  // final row passes writing the bit-reversed order
         registry()[Key{LT, LI, COL, SINGLE, false, 32}] = &launch<LT, LI, COL, SINGLE, false, 32>;
@@ -1230,6 +1279,21 @@ class FftExecutor final : public Executor {
         mapping_json = w.str();
     }
     std::size_t workspace_bytes() const override { return workspace_; }
+    // Makes a one-pass plan of the static lowering read (forward) or write
+    // (inverse) rows of `len` elements; false where it has no such kernel.
+    bool use_ragged_rows(std::uint64_t len, std::uint64_t in_pitch, std::uint64_t out_pitch) {
+        const int m = int(r_.log_n);
+        if (steps_.size() != 1 || m > 14 || r_.pitched || len < 1 || len > r_.n) return false;
+        if (steps_[0].fn != lookup(Key{m, single_li(m), false, true, r_.inverse})) return false;
+        // 32-bit byte offsets within a tile of several rows (and below the
+        // offset that stands for an absent element).
+        if ((r_.inverse ? out_pitch : in_pitch) >= (std::uint64_t{1} << (28 - single_li(m)))) return false;
+        steps_[0].fn = find(Key{m, single_li(m), false, true, r_.inverse, 64});
+        steps_[0].args.in_pitch = in_pitch;
+        steps_[0].args.out_pitch = out_pitch;
+        steps_[0].args.row_len = std::uint32_t(len);
+        return true;
+    }
     void execute(const void* in, void* out, void* ws, hipStream_t stream) override {
         require(steps_.size() < 2 || ws != nullptr, "two-pass FFT needs a workspace");
         for (const auto& s : steps_) {
@@ -1447,6 +1511,11 @@ class FftRank2ColumnsExecutor final : public Executor {
 };
 
 }  // namespace
+
+bool fft_use_ragged_rows(Executor& plan, std::uint64_t len, std::uint64_t in_pitch, std::uint64_t out_pitch) {
+    auto* fft = dynamic_cast<FftExecutor*>(&plan);
+    return fft != nullptr && fft->use_ragged_rows(len, in_pitch, out_pitch);
+}
 
 bool fft_rows_transposed_available(const Request& r, std::uint32_t l1) {
     const int l2 = int(r.log_n);

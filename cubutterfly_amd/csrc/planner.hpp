@@ -23,6 +23,11 @@ std::vector<std::string> fwht_candidates(const Request& r);
 std::string fwht_mfma_name();
 bool fwht_mfma_covers(const Request& r);
 std::unique_ptr<Executor> make_fwht_mfma_executor(const Request& r);
+// Makes a one-pass FFT plan of packed natural-order rows take forward input or
+// inverse output rows of only `len` of the n elements, in_pitch / out_pitch
+// elements apart (the other side packed): zeros read, surplus dropped. False,
+// the plan unchanged, where no kernel covers it.
+bool fft_use_ragged_rows(Executor& plan, std::uint64_t len, std::uint64_t in_pitch, std::uint64_t out_pitch);
 // FFTs (r.log_n points) of the rows of row-major 2^l1 x 2^(r.log_n) blocks
 // (r.batch rows in all), each block's result stored transposed; null where
 // no kernel covers the shape.
