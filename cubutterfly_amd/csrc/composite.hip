@@ -268,21 +268,39 @@ __global__ __launch_bounds__(kThreads) void fwht_columns_kernel(const float* src
     }
 }
 
+// Consecutive columns per lane: up to 4 of at most 8 rows, one of more (FP16
+// results: as many as the registers hold, so a lane's halves make whole words).
+// A pass is bound by the loads in flight, and one column of 16 or more rows per
+// lane means more waves: the pass alone, FP32 rows of 2^18 points, 64 rows with
+// 2 / 1 columns a lane: 8 MiB 6.9 / 4.5 us, 40 MiB 17.6 / 13.7, 64 MiB 21.6 /
+// 20.7; 32 rows with 4 / 1: 5.1 / 3.7, 14.8 / 13.3, 21.8 / 19.6; 16 rows: 3.9 /
+// 3.4, 13.0 / 12.5, 19.0 / 18.4; but 8 rows with 4 / 2: 3.5 / 3.4, 12.2 / 12.5,
+// 17.7 / 18.2. 32 rows from 64 MiB on keep 4 columns, which were as fast there
+// behind the row pass (2^17-point rows: 50.9 / 52.0 us for both passes).
+template <int LOG_L, bool NARROW>
+constexpr int column_vector() {
+    return NARROW ? (LOG_L <= 5 ? 4 : LOG_L == 6 ? 2 : 1) : LOG_L <= 3 || LOG_L == 5 ? 4 : 1;
+}
+
+// `vec`: the widest vector the pointers' alignment allows.
 template <int LOG_L, bool NARROW>
 void launch_fwht_columns_rows(const float* src, void* dst, std::uint64_t count, std::uint32_t log_cols, int vec,
                               float scale, bool apply_scale, float out_scale, hipStream_t stream) {
+    constexpr int kVec = column_vector<LOG_L, NARROW>();
+    vec = std::min(vec, kVec);
+    if (!NARROW && LOG_L == 5 && count < (std::uint64_t{1} << 24)) vec = 1;
     const std::uint64_t vectors = count >> (LOG_L + (vec == 4 ? 2 : vec == 2 ? 1 : 0));
     const std::uint64_t blocks = (vectors + kThreads - 1) / kThreads;
     require(blocks < (std::uint64_t{1} << 31), "FWHT column pass grid too large");
     const dim3 grid{unsigned(blocks)}, block{kThreads};
-    if constexpr (LOG_L <= 5) {
+    if constexpr (kVec >= 4) {
         if (vec == 4) {
             hipLaunchKernelGGL((fwht_columns_kernel<LOG_L, 4, NARROW>), grid, block, 0, stream, src, dst, vectors,
                                log_cols, scale, int(apply_scale), out_scale);
             return;
         }
     }
-    if constexpr (LOG_L <= 6) {
+    if constexpr (kVec >= 2) {
         if (vec == 2) {
             hipLaunchKernelGGL((fwht_columns_kernel<LOG_L, 2, NARROW>), grid, block, 0, stream, src, dst, vectors,
                                log_cols, scale, int(apply_scale), out_scale);
@@ -310,8 +328,7 @@ void launch_fwht_columns_of(const float* src, void* dst, std::uint64_t count, st
 
 // Column pass over `count` FP32 elements (G blocks of 2^log_rows x
 // 2^log_cols), src == dst allowed; with `narrow_out`, the results go there as
-// FP16 (narrow_scaled(x, out_scale)) instead. The widest vector both
-// pointers' alignment and the register budget allow.
+// FP16 (narrow_scaled(x, out_scale)) instead.
 void launch_fwht_columns(const float* src, float* dst, std::uint64_t count, std::uint32_t log_rows,
                          std::uint32_t log_cols, float scale, bool apply_scale, hipStream_t stream,
                          __half* narrow_out = nullptr, float out_scale = 1.0f) {
@@ -325,8 +342,6 @@ void launch_fwht_columns(const float* src, float* dst, std::uint64_t count, std:
         const auto d = reinterpret_cast<std::uintptr_t>(dst);
         vec = std::min(vec, d % 16 == 0 ? 4 : d % 8 == 0 ? 2 : 1);
     }
-    if (log_rows == 6) vec = std::min(vec, 2);
-    if (log_rows == 7) vec = 1;
     if (narrow_out)
         launch_fwht_columns_of<true>(src, narrow_out, count, log_rows, log_cols, vec, scale, apply_scale, out_scale,
                                      stream);
