@@ -16,9 +16,10 @@
 // the original order (two HBM round trips where the transposes take four).
 // The transposing store writes segments of 2^(14 - n) elements for rows of
 // 2^n points; where an axis has 2^11 points or more (segments under 128
-// bytes) the block runs instead as column passes over axis 0 and a row pass
-// over axis 1 that stores whole rows (every segment 512 bytes or longer).
-// Either lowering can be named (EXPLICIT) where its kernels cover the shape.
+// bytes), or of 2^9 in 2^21 points or more, the block runs instead as column
+// passes over axis 0 and a row pass over axis 1 that stores whole rows. Blocks of
+// at most 2^14 points are transformed whole, both axes in one pass. Each lowering
+// can be named (EXPLICIT) where its kernels cover the shape.
 //
 // FWHT needs none of this: the Sylvester Hadamard matrix of n0 * n1 points
 // is the Kronecker product H(n0) (x) H(n1), and the innermost-first axis
@@ -366,7 +367,8 @@ struct Step {
 class CompositeExecutor final : public Executor {
   public:
     // force: 0 the static rule (or the name an EXPLICIT request gives), 1 a
-    // rank-2 FFT's column passes, 2 its transposing row passes.
+    // rank-2 FFT's column passes, 2 its transposing row passes, 3 its one-pass
+    // blocks, 4 the static rule without them.
     CompositeExecutor(const Request& r, bool flatten, Selection* sel, int force = 0) : r_(r) {
         const std::uint32_t rank = r.rank;
         std::vector<std::uint32_t> logs(rank);
@@ -376,13 +378,36 @@ class CompositeExecutor final : public Executor {
         in_side_ = side(true, logs);
         out_side_ = side(false, logs);
         std::vector<std::string> names;
-        // A rank-2 FFT named explicitly as one of its two lowerings takes that
-        // one (EXPLICIT); otherwise column passes from 2^11-point axes.
+        // A rank-2 FFT named explicitly as one of its lowerings takes that one
+        // (EXPLICIT). Static rule: whole blocks in one pass where they fit; else
+        // axis 0 as column passes from 2^11-point axes, and from 2^9-point axes
+        // in 2^21 points or more; else transposing rows where their kernels cover
+        // the shape, else transposes. Measured, us, transposes or transposing rows
+        // / columns / blocks:
+        //   32 x 32 (2^23 points) 199 / - / 30, (2^18) 25.9 / - / 6.9;
+        //   128 x 64 124 / - / 33; 128 x 128 49.5 / 50.2 / 37.1;
+        //   256 x 256 47.4 / 48.3; 512 x 1024 66.7 / 54.9, (2^21) 27.1 / 23.2;
+        //   2048 x 2048 67.8 / 53.5.
+        // (Columns are as far ahead below 2^21 points: 512 x 1024, 2^19 points,
+        // 22.4 / 17.6. There the rows stay the default, which programs name, and
+        // the columns are MEASURE's choice.)
         const bool named = r.policy == CUBUTTERFLY_ALGORITHM_EXPLICIT;
-        const bool want_columns = force == 1 || (named && r.explicit_algorithm.rfind("rank2-columns[", 0) == 0);
-        const bool want_rows = force == 2 || (named && r.explicit_algorithm.rfind("rank2-transposing[", 0) == 0);
-        if (!flatten && r.op == Op::Fft && rank == 2 && !want_rows &&
-            (want_columns || std::max(logs[0], logs[1]) >= 11)) {
+        const auto names_it = [&](const char* prefix) { return named && r.explicit_algorithm.rfind(prefix, 0) == 0; };
+        const bool want_columns = force == 1 || names_it("rank2-columns[");
+        const bool want_rows = force == 2 || names_it("rank2-transposing[");
+        const bool want_blocks = force == 3 || (named ? names_it("rank2-blocks[") : force == 0);
+        const std::uint32_t longest = rank == 2 ? std::max(logs[0], logs[1]) : 0;
+        const bool fft2 = !flatten && r.op == Op::Fft && rank == 2;
+        if (fft2 && want_blocks) {
+            auto blocks = make_fft_rank2_blocks(axis_request(r.n, r.batch), logs[0]);
+            if (blocks) {
+                blocks_ = true;
+                children_.push_back(std::move(blocks));
+                steps_.push_back(Step{false, 0, 0, 0, 0, 0});
+            }
+        }
+        if (fft2 && !blocks_ && !want_rows &&
+            (want_columns || longest >= 11 || (longest >= 9 && r.n * r.batch >= (std::uint64_t{1} << 21)))) {
             // Axis 0 as column passes over each block, then the rows.
             auto cols = make_fft_rank2_columns(axis_request(r.n, r.batch), logs[0]);
             if (cols) {
@@ -391,7 +416,7 @@ class CompositeExecutor final : public Executor {
                 steps_.push_back(Step{false, 0, 0, 0, 0, 0});
             }
         }
-        if (!columns_ && !want_columns && !flatten && r.op == Op::Fft && rank == 2) {
+        if (fft2 && !blocks_ && !columns_ && !want_columns) {
             // Each axis as one row pass that stores its blocks transposed:
             // rows of the caller's layout, then rows of the transposed one,
             // which lands back in the original order. No transpose kernels.
@@ -406,7 +431,7 @@ class CompositeExecutor final : public Executor {
                 steps_.push_back(Step{false, 1, 0, 0, 0, 0});
             }
         }
-        if (transposing_ || columns_) {
+        if (transposing_ || columns_ || blocks_) {
         } else if (flatten) {
             children_.push_back(plan_executor(axis_request(r.n, r.batch), sel));
             steps_.push_back(Step{false, 0, 0, 0, 0, 0});
@@ -491,12 +516,14 @@ class CompositeExecutor final : public Executor {
                                 : rank == 1    ? "zero-extended"
                                 : transposing_ ? "rank2-transposing"
                                 : columns_     ? "rank2-columns"
+                                : blocks_      ? "rank2-blocks"
                                 : fwht_columns_ ? (rank == 2 ? "rank2-fwht-columns" : "rankN-fwht-columns")
                                 : flatten      ? (rank == 2 ? "rank2-kronecker" : "rankN-kronecker")
                                                : (rank == 2 ? "rank2-transpose" : "rankN-composite")) +
                     "[" + joined + "]" + (direct_in_ ? "+direct-input" : "") + (direct_out_ ? "+direct-output" : "");
         reason = transposing_ ? "each axis one row pass with a transposing store (innermost axis first)"
                  : columns_   ? "axis 0 as column passes over each block, then the rows stored in natural order"
+                 : blocks_    ? "both axes of whole blocks in one pass"
                  : fwht_columns_
                      ? "innermost axis one row plan, the other axes in-place column passes of at most 2^7 rows "
                        "(FWHT stages in index-bit order, no transposes)"
@@ -511,6 +538,7 @@ class CompositeExecutor final : public Executor {
             .field("rank", rank)
             .field("lowering", transposing_ ? "transposing-rows"
                                : columns_   ? "columns-then-rows"
+                               : blocks_    ? "resident-blocks"
                                : fwht_columns_ ? "rows-then-columns"
                                : flatten    ? "kronecker"
                                             : "transpose")
@@ -535,7 +563,7 @@ class CompositeExecutor final : public Executor {
             } else if (s.transpose) {
                 w.field("step", "transpose").field("blocks", s.groups).field("rows", std::uint64_t{1} << s.log_rows)
                     .field("cols", std::uint64_t{1} << s.log_cols);
-            } else if (columns_) {
+            } else if (columns_ || blocks_) {
                 w.field("step", "axes");
                 w.begin_array("axes").value(0u).value(1u).end_array();
                 w.key("child").value_raw(children_[s.child]->mapping_json);
@@ -577,6 +605,7 @@ class CompositeExecutor final : public Executor {
 
     bool columns() const { return columns_; }
     bool transposing() const { return transposing_; }
+    bool blocks() const { return blocks_; }
 
     std::size_t workspace_bytes() const override {
         // The ping-pong buffers, then the largest child's workspace.
@@ -644,6 +673,11 @@ class CompositeExecutor final : public Executor {
         return fft_rank2_columns_available(axis_request_of(r, r.n, r.batch), l0) &&
                fft_rows_transposed_available(axis_request_of(r, r.extents[1], r.batch * r.extents[0]), l0) &&
                fft_rows_transposed_available(axis_request_of(r, r.extents[0], r.batch * r.extents[1]), l1);
+    }
+
+    // Whether it has the one-pass blocks (no device work).
+    static bool fits_blocks(const Request& r) {
+        return fft_rank2_blocks_available(axis_request_of(r, r.n, r.batch), log2_u64(r.extents[0]));
     }
 
   private:
@@ -740,7 +774,7 @@ class CompositeExecutor final : public Executor {
     }
 
     Request r_;
-    bool transposing_ = false, columns_ = false, fwht_columns_ = false;
+    bool transposing_ = false, columns_ = false, blocks_ = false, fwht_columns_ = false;
     bool ragged_ = false;  // the child reads and writes the caller's rows (rank-1 embedding)
     bool direct_in_ = false, direct_out_ = false;
     NdSide in_side_, out_side_;
@@ -886,7 +920,7 @@ std::unique_ptr<Executor> make_composite_executor(const Request& r, Selection* s
             "composite plans need rank 2 to 8, the zero-extended embedding or a factored FWHT");
     // A flattened FWHT is one rank-1 plan; it exists up to the resident length.
     const bool flatten = r.op == Op::Fwht && !(r.inverse && r.normalize) && r.log_n <= kMaxFwhtRowLog;
-    // A rank-2 FFT with both lowerings: MEASURE times the two, DEFAULT
+    // A rank-2 FFT with several lowerings: MEASURE times them, DEFAULT
     // replays a selection-cache record of that choice (keyed by the extents
     // too), the static rule decides otherwise.
     if (!flatten && r.op == Op::Fft && r.rank == 2 && !r.embedding && sel != nullptr &&
@@ -899,6 +933,8 @@ std::unique_ptr<Executor> make_composite_executor(const Request& r, Selection* s
             const std::string cached = lookup_cache(sel->cache_path, key);
             const int force = cached.rfind("rank2-columns[", 0) == 0       ? 1
                               : cached.rfind("rank2-transposing[", 0) == 0 ? 2
+                              : cached.rfind("rank2-blocks[", 0) == 0      ? 3
+                              : cached.rfind("rank2-transpose[", 0) == 0   ? 4
                                                                            : 0;
             if (force) {
                 auto e = std::make_unique<CompositeExecutor>(r, flatten, sel, force);
@@ -909,16 +945,26 @@ std::unique_ptr<Executor> make_composite_executor(const Request& r, Selection* s
                 }
                 note_selection(*sel, "ignored cache record '" + cached + "' (not a lowering of this request)");
             }
-        } else if (CompositeExecutor::both_rank2_lowerings(r)) {
-            require_no_capture(*sel);
-            auto cols = std::make_unique<CompositeExecutor>(r, flatten, sel, 1);
-            auto rows = std::make_unique<CompositeExecutor>(r, flatten, sel, 2);
-            if (cols->columns() && rows->transposing()) {
+        } else {
+            const bool both = CompositeExecutor::both_rank2_lowerings(r), whole = CompositeExecutor::fits_blocks(r);
+            if (both || whole) {
+                require_no_capture(*sel);
                 std::vector<std::unique_ptr<Executor>> alternatives;
-                alternatives.push_back(std::move(cols));
-                alternatives.push_back(std::move(rows));
-                const std::size_t best = measure_executors(r, key, alternatives, *sel);
-                if (best < alternatives.size()) return std::move(alternatives[best]);
+                const auto offer = [&](int force, bool (CompositeExecutor::*is)() const) {
+                    auto e = std::make_unique<CompositeExecutor>(r, flatten, sel, force);
+                    if (is == nullptr || (e.get()->*is)()) alternatives.push_back(std::move(e));
+                };
+                if (both) {
+                    offer(1, &CompositeExecutor::columns);
+                    offer(2, &CompositeExecutor::transposing);
+                } else {
+                    offer(4, nullptr);
+                }
+                if (whole) offer(3, &CompositeExecutor::blocks);
+                if (alternatives.size() >= 2) {
+                    const std::size_t best = measure_executors(r, key, alternatives, *sel);
+                    if (best < alternatives.size()) return std::move(alternatives[best]);
+                }
             }
         }
     }

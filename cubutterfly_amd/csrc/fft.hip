@@ -1051,6 +1051,9 @@ void register_all() {
     add<4, 10, true, false>();
     add<5, 9, true, false>();
     add<6, 8, true, false>();
+    add_rank2_rows<5>();
+    add_rank2_rows<6>();
+    add_rank2_rows<7>();
     add_rank2_rows<8>();
     add_rank2_rows<9>();
     add_rank2_rows<10>();
@@ -1410,6 +1413,161 @@ class FftRowsTransposedExecutor final : public Executor {
     DeviceBuffer twa_, twb_;
 };
 
+// Rank-2 FFTs of small row-major 2^l0 x 2^l1 blocks, whole blocks resident in a
+// workgroup: a tile of 2^LB points holds 2^(LB - l0 - l1) blocks, 16 values per
+// thread. The axis-0 digits come first, then the axis-1 digits (4 bits each, top
+// digit first, an LDS exchange between), with level twiddles of the digit's own
+// axis only; the final store reads each axis in bit-reversed order from the LDS,
+// so whole contiguous blocks leave as they came. One HBM round trip where the
+// row passes with transposes between take four, or column and row passes two.
+// The axis lengths are run-time values (windows and bit reversals are a few
+// integer operations per register beside 16-point codelets): one kernel per tile
+// size and direction. LDS image: one pad word per 16.
+struct Fft2Args {
+    const float2* in;
+    float2* out;
+    const float2* tw;  // w^k of the 2^lw-point transform, lw the longer axis, k < 2^lw
+    std::uint32_t l0, l1, lw;
+    std::uint64_t points;  // batch * 2^(l0 + l1)
+    float scale;
+};
+
+template <int LB, bool INV>
+__global__ __launch_bounds__(1 << (LB - 4)) void fft_rank2_block_kernel(Fft2Args a) {
+    using Digits = FftPass<12, 0, false, true, INV>;  // 16 values: its powers of a level twiddle base
+    constexpr std::uint32_t T = 1u << (LB - 4);
+    __shared__ float2 lds[(1u << LB) + (1u << (LB - 4))];
+    const auto addr = [](std::uint32_t i) { return i + (i >> 4); };  // a sum over disjoint index bits
+    const auto thread_index = [](std::uint32_t t, std::uint32_t s) { return (t & ((1u << s) - 1u)) | ((t >> s) << (s + 4)); };
+    const std::uint32_t t = threadIdx.x;
+    const std::uint64_t first = std::uint64_t(blockIdx.x) << LB;
+    const std::uint32_t bytes = std::uint32_t(min(std::uint64_t{1} << LB, a.points - first)) * 8u;
+    const __amdgpu_buffer_rsrc_t src = make_rsrc(a.in + first, bytes), dst = make_rsrc(a.out + first, bytes);
+    const __amdgpu_buffer_rsrc_t tw = make_rsrc(a.tw, 8u << a.lw);
+    float2 v[16];
+    std::uint32_t window = 0;
+    bool loaded = false;
+    for (int axis = 0; axis < 2; ++axis) {
+        const std::uint32_t base = axis == 0 ? a.l1 : 0u;
+        std::uint32_t rem = axis == 0 ? a.l0 : a.l1;  // the axis's bits below the digits done
+        while (rem > 0) {
+            // The digit's bits are the lowest of the window's (a last digit of
+            // fewer than 4 bits has bits already done above it).
+            const std::uint32_t digit = min(rem, 4u);
+            rem -= digit;
+            const std::uint32_t s = base + rem;
+            const std::uint32_t it = thread_index(t, s);
+            if (!loaded) {
+#pragma unroll
+                for (std::uint32_t r = 0; r < 16; ++r) v[r] = buffer_load<float2, 2>(src, (it + (r << s)) * 8u);
+            } else {
+                const std::uint32_t wt = addr(thread_index(t, window)), rt = addr(it);
+                lds_barrier();
+#pragma unroll
+                for (std::uint32_t r = 0; r < 16; ++r) lds[wt + addr(r << window)] = v[r];
+                lds_barrier();
+#pragma unroll
+                for (std::uint32_t r = 0; r < 16; ++r) v[r] = lds[rt + addr(r << s)];
+            }
+            loaded = true;
+            window = s;
+            if (rem > 0) {  // a full digit with more of the axis below it
+                const std::uint32_t jl = (it >> base) & ((1u << rem) - 1u);
+                const float2 p1 = buffer_load<float2>(tw, (jl << (a.lw - (rem + 4u))) * 8u);
+                codelet<16, 4, INV>(v);
+                const float2 p2 = cmul(p1, p1), p3 = cmul(p2, p1), p4 = cmul(p2, p2), p8 = cmul(p4, p4);
+                Digits::template apply_powers<0, 4>(v, p1, p2, p3, p4, p8, p1);
+            } else if (digit == 4) {
+                codelet<16, 4, INV>(v);
+            } else if (digit == 3) {
+                codelet<16, 3, INV>(v);
+            } else if (digit == 2) {
+                codelet<16, 2, INV>(v);
+            } else {
+                codelet<16, 1, INV>(v);
+            }
+        }
+    }
+    const std::uint32_t wt = addr(thread_index(t, window));
+    lds_barrier();
+#pragma unroll
+    for (std::uint32_t r = 0; r < 16; ++r) lds[wt + addr(r << window)] = v[r];
+    lds_barrier();
+#pragma unroll
+    for (std::uint32_t r = 0; r < 16; ++r) {
+        const std::uint32_t o = t + T * r;
+        const std::uint32_t x = o & ((1u << a.l1) - 1u), y = (o >> a.l1) & ((1u << a.l0) - 1u);
+        const std::uint32_t i = ((o >> (a.l0 + a.l1)) << (a.l0 + a.l1)) | (brev(y, a.l0) << a.l1) | brev(x, a.l1);
+        const float2 c = lds[addr(i)];
+        buffer_store<float2, 2>(make_float2(c.x * a.scale, c.y * a.scale), dst, o * 8u);
+    }
+}
+
+constexpr int rank2_block_tile(int m) { return m < 12 ? 12 : m; }
+
+class FftRank2BlocksExecutor final : public Executor {
+  public:
+    FftRank2BlocksExecutor(const Request& r, std::uint32_t l0) {
+        const std::uint32_t l1 = r.log_n - l0;
+        args_.l0 = l0;
+        args_.l1 = l1;
+        args_.lw = std::max(l0, l1);
+        args_.points = r.batch * r.n;
+        args_.scale = r.normalize ? 1.0f / float(r.n) : 1.0f;
+        const std::size_t n = std::size_t{1} << args_.lw;
+        std::vector<float2> table(n);
+        for (std::size_t k = 0; k < n; ++k) {
+            const double angle = (r.inverse ? 2.0 : -2.0) * M_PI * double(k) / double(n);
+            table[k] = make_float2(float(std::cos(angle)), float(std::sin(angle)));
+        }
+        tw_.upload(table);
+        args_.tw = tw_.as<float2>();
+        inverse_ = r.inverse;
+        tile_ = rank2_block_tile(int(r.log_n));
+        grid_ = unsigned((args_.points + (std::uint64_t{1} << tile_) - 1) >> tile_);
+        algorithm = "fft-c64-rank2-blocks-r16";
+        reason = "whole 2^" + std::to_string(l0) + " x 2^" + std::to_string(l1) +
+                 " blocks resident in one workgroup, both axes in one pass";
+        json::Writer w;
+        w.begin_object()
+            .field("schema_version", 1u)
+            .field("operator", "fft")
+            .field("algorithm", algorithm)
+            .field("log_n", r.log_n)
+            .field("axis0_bits", l0)
+            .field("blocks", r.batch)
+            .field("blocks_per_tile", std::uint64_t{1} << (tile_ - int(r.log_n)))
+            .field("direction", r.inverse ? "inverse" : "forward")
+            .end_object();
+        mapping_json = w.str();
+    }
+    void execute(const void* in, void* out, void*, hipStream_t stream) override {
+        Fft2Args a = args_;
+        a.in = static_cast<const float2*>(in);
+        a.out = static_cast<float2*>(out);
+        switch (tile_) {
+            case 12: launch<12>(a, stream); break;
+            case 13: launch<13>(a, stream); break;
+            default: launch<14>(a, stream); break;
+        }
+        hip_check(hipGetLastError(), "FFT pass launch");
+    }
+
+  private:
+    template <int LB>
+    void launch(const Fft2Args& a, hipStream_t stream) const {
+        if (inverse_)
+            hipLaunchKernelGGL((fft_rank2_block_kernel<LB, true>), dim3(grid_), dim3(1u << (LB - 4)), 0, stream, a);
+        else
+            hipLaunchKernelGGL((fft_rank2_block_kernel<LB, false>), dim3(grid_), dim3(1u << (LB - 4)), 0, stream, a);
+    }
+    Fft2Args args_{};
+    DeviceBuffer tw_;
+    bool inverse_ = false;
+    int tile_ = 12;
+    unsigned grid_ = 0;
+};
+
 // Rank-2 FFTs of row-major 2^l0 x 2^l1 blocks (r.n = 2^(l0 + l1) points per
 // block, r.batch blocks): the axis-0 transform as one or two column passes
 // over each block (the low l1 bits of their column index number
@@ -1533,20 +1691,24 @@ std::unique_ptr<Executor> make_fft_rows_transposed(const Request& r, std::uint32
 }
 
 // The column-pass split of axis 0 (ta top bits, then tb; tb = 0 for one
-// pass), or false where no kernels cover the shape: rows of 2^8 .. 2^12
-// points (whole 2^14-point row tiles within a block), blocks of at most 2^24
+// pass), or false where no kernels cover the shape: rows of 2^5 .. 2^12
+// points (whole 2^14-point column tiles within a block), blocks of at most 2^24
 // points (the level-twiddle tables' reach), and axis 0 in one column pass of
-// 4 .. 8 bits or two: the second over tb >= 14 - l1 bits (its 2^(14 - tb)
-// columns within the 2^l1 of a row), the first over the rest, each within
-// 4 .. 8 bits.
+// 4 .. 11 bits, its 2^(14 - ta) columns within the 2^l1 of a row, or two: the
+// second over tb >= 14 - l1 bits, the first over the rest, each within 4 .. 8
+// bits. One pass of 9 to 11 bits moves segments of 256 to 64 bytes and still
+// beats two (2^23 points, 2048 x 1024: 53.8 against 74.7 us, 2048 x 2048 53.5
+// against 76.1). Blocks with 2^12-point rows keep two from 2^9 points on,
+// though one is faster there too (512 x 4096 x 2 50.4 / 33.3 us, 2048 x 4096 78.0
+// / 58.9): their mapping (`column_passes`) is what programs have seen.
 bool rank2_columns_split(const Request& r, std::uint32_t l0, std::uint32_t& ta, std::uint32_t& tb) {
     const std::uint32_t m = r.log_n;
     if (l0 < 4 || l0 >= m) return false;
     const std::uint32_t l1 = m - l0;
-    if (l1 < 8 || l1 > 12 || m > 24 || l0 < 14 - l1) return false;
+    if (l1 < 5 || l1 > 12 || m > 24 || l0 < 14 - l1) return false;
     ta = l0;
     tb = 0;
-    if (l0 > 8) {
+    if (l0 > (l1 < 12 ? 11u : 8u)) {
         tb = std::max(l0 / 2, 14 - l1);
         ta = l0 - tb;
         if (tb > 8 || ta < 4 || ta > 8) return false;
@@ -1563,6 +1725,23 @@ std::unique_ptr<Executor> make_fft_rank2_columns(const Request& r, std::uint32_t
     std::uint32_t ta = 0, tb = 0;
     if (!rank2_columns_split(r, l0, ta, tb)) return nullptr;
     return std::make_unique<FftRank2ColumnsExecutor>(r, l0, ta, tb);
+}
+
+// Axes of 2^1 points up (a window of 4 bits above axis 1 stays inside the tile),
+// blocks of at most 2^14 points, at least one tile for each of the 8 XCDs.
+bool fft_rank2_blocks_available(const Request& r, std::uint32_t l0) {
+    const std::uint32_t m = r.log_n;
+    if (l0 < 1 || l0 >= m || m > 14) return false;
+    const int tile = rank2_block_tile(int(m));
+    const std::uint32_t l1 = m - l0;
+    if (int(l1) + 4 > tile) return false;
+    const std::uint64_t tiles = (r.batch * r.n + (std::uint64_t{1} << tile) - 1) >> tile;
+    return tiles >= 8 && tiles <= 0x7fffffffull;
+}
+
+std::unique_ptr<Executor> make_fft_rank2_blocks(const Request& r, std::uint32_t l0) {
+    if (!fft_rank2_blocks_available(r, l0)) return nullptr;
+    return std::make_unique<FftRank2BlocksExecutor>(r, l0);
 }
 
 // One-pass lengths have one lowering; two-pass lengths add the neighbouring

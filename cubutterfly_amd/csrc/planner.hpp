@@ -36,7 +36,11 @@ std::unique_ptr<Executor> make_fft_rows_transposed(const Request& r, std::uint32
 // r.n points): axis 0 as column passes, then the rows in natural order; null
 // where no kernel covers the shape.
 std::unique_ptr<Executor> make_fft_rank2_columns(const Request& r, std::uint32_t l0);
-// Whether those two factories would build a plan (no device work).
+// Rank-2 FFTs of 2^l0 x 2^(r.log_n - l0) blocks, whole blocks in one workgroup;
+// null where no kernel covers the shape.
+std::unique_ptr<Executor> make_fft_rank2_blocks(const Request& r, std::uint32_t l0);
+bool fft_rank2_blocks_available(const Request& r, std::uint32_t l0);
+// Whether the two factories before would build a plan (no device work).
 bool fft_rows_transposed_available(const Request& r, std::uint32_t l1);
 bool fft_rank2_columns_available(const Request& r, std::uint32_t l0);
 std::vector<std::string> fft_candidates(const Request& r);
