@@ -507,22 +507,22 @@ struct Pass {
     static constexpr std::uint32_t kPolyBytes = std::uint32_t(sizeof(W)) << kLogN;
     using L = Lds<COL, COL && (PIN || POUT), LT, LI, !COL && sizeof(W) == 4 && LT == 8 && LI <= 5,
                   SINGLE && LT >= kLongRow ? int(sizeof(W)) : 0>;
-    // Stores of two-pass inverse (Gentleman-Sande) tiles write through the L2
-    // (sc0 sc1), so the end-of-kernel write-back has little left to flush;
-    // measured 5-6% faster per C2 / C4 step. Forward passes keep write-back
-    // stores: write-through made them slower (partial-line segments that
-    // the L2 would otherwise merge).
-    // (Nontemporal final stores measured slower for C4, whose bit-reversed
-    // output lands in 8-byte segments: 60.6 -> 71-73 us.) Forward column
-    // passes whose tiles write whole 128-byte lines per row (u32 32-column,
-    // u64 16-column tiles) store the intermediate nontemporally: C4 56.5 ->
-    // 54.9 us, C2 unchanged. Forward row passes that stage their stores
-    // (natural output through the LDS permutation, or native output through
-    // the wave's own rows, kStagedAux) write through as well: C2 38.6 ->
-    // 37.3 us, C4 54.2 -> 52.0 us.
-    static constexpr int kStoreAux = (!CT && !SINGLE) || (CT && !SINGLE && !COL && POUT) ? 17
-                                     : (COL && CT && !SINGLE && (sizeof(W) << LI) >= 128) ? 2
-                                                                                          : 0;
+    // Stores of two-pass tiles write through the L2 (sc0 sc1), so the
+    // end-of-kernel write-back has little left to flush: inverse passes (5-6%
+    // of a C2 / C4 step), forward row passes that stage their stores (natural
+    // output through the LDS permutation, or native output through the wave's
+    // own rows, kStagedAux: C2 38.6 -> 37.3 us, C4 54.2 -> 52.0), and forward
+    // column passes whose tiles write whole 128-byte lines per row (u32
+    // 32-column, u64 16-column tiles), which the row pass then finds in the
+    // Infinity Cache where nontemporal stores left it to memory: forward and
+    // inverse of u32 2^16 x 64 36.3 -> 35.0 us, x 128 73.3 -> 65.9; u64 2^16 x 32
+    // 41.9 -> 41.1, x 64 76.1 -> 72.3. Forward column passes of narrower tiles keep
+    // write-back stores: write-through made them slower (partial-line segments
+    // that the L2 would otherwise merge). (Nontemporal final stores measured
+    // slower for C4, whose bit-reversed output lands in 8-byte segments: 60.6 ->
+    // 71-73 us.)
+    static constexpr int kStoreAux =
+        !SINGLE && (!CT || (COL ? (sizeof(W) << LI) >= 128 : POUT)) ? 17 : 0;
     // A register window starting at tile bit S <= 6 leaves tile bits 10 and up
     // to the wave index (phase_index: thread bits from 6 up are tile bits from
     // 10 up), so an exchange between two such windows never leaves a wave: all
@@ -544,6 +544,12 @@ struct Pass {
     // as contiguous runs and moving them into the phase-0 layout through the
     // wave's rows, measured no faster: C4 52.7 against 52.0-52.2 us.)
     static constexpr int kPer = 16 / int(sizeof(W));  // words per 16-byte access
+    // Twiddle chunks one phase ahead: u32 two-pass tiles have the registers (95 of
+    // the 128 that 4 waves per SIMD allow, and a batch of 64 fills no more) and
+    // gain the L2 latency of each phase: u32 2^16 x 64 forward and inverse 35.3 ->
+    // 34.3 us, x 128 66.4 -> 63.3. u64 tiles lose occupancy for it (2^16 x 32 41.7 ->
+    // 43.3 us), and one-pass tiles run more waves per SIMD.
+    static constexpr bool kAhead = sizeof(W) == 4 && !SINGLE && !BARRETT && kPhases <= 3;
 
     // Staged store run: lane l of wave w moves tile elements g0 + 64 kPer k + e
     // (e < kPer), g0 = 1024 w + kPer l. The thread, lane and register parts
@@ -927,21 +933,30 @@ struct Pass {
                 }
             }
         }
+        // A later phase's chunk loads during the exchange before it (or, kAhead,
+        // one phase earlier: before the butterflies of the phase before it).
+        Chunk<1> c1;
+        Chunk<2> c2;
+        Chunk<3> c3;
+        if constexpr (kAhead) {
+            load_chunk<1>(c1, a, tl, t, twiddles(a, d));
+            __builtin_amdgcn_sched_barrier(0);
+        }
         stages<0>(v, c0, d);
         if constexpr (kPhases > 1) {
-            Chunk<1> c1;
-            exchange<tile_window<0>(), tile_window<1>()>(v, lds, t,
-                                                         [&] { load_chunk<1>(c1, a, tl, t, twiddles(a, d)); });
+            exchange<tile_window<0>(), tile_window<1>()>(v, lds, t, [&] {
+                if constexpr (kAhead) load_chunk<2>(c2, a, tl, t, twiddles(a, d));
+                else load_chunk<1>(c1, a, tl, t, twiddles(a, d));
+            });
             stages<1>(v, c1, d);
         }
         if constexpr (kPhases > 2) {
-            Chunk<2> c2;
-            exchange<tile_window<1>(), tile_window<2>()>(v, lds, t,
-                                                         [&] { load_chunk<2>(c2, a, tl, t, twiddles(a, d)); });
+            exchange<tile_window<1>(), tile_window<2>()>(v, lds, t, [&] {
+                if constexpr (!kAhead) load_chunk<2>(c2, a, tl, t, twiddles(a, d));
+            });
             stages<2>(v, c2, d);
         }
         if constexpr (kPhases > 3) {
-            Chunk<3> c3;
             exchange<tile_window<2>(), tile_window<3>()>(v, lds, t,
                                                          [&] { load_chunk<3>(c3, a, tl, t, twiddles(a, d)); });
             stages<3>(v, c3, d);
