@@ -16,7 +16,7 @@
 // the original order (two HBM round trips where the transposes take four).
 // The transposing store writes segments of 2^(14 - n) elements for rows of
 // 2^n points; where an axis has 2^11 points or more (segments under 128
-// bytes), or of 2^9 in 2^21 points or more, the block runs instead as column
+// bytes), or axis 0 2^9 in 2^21 points or more, the block runs instead as column
 // passes over axis 0 and a row pass over axis 1 that stores whole rows. Blocks of
 // at most 2^14 points are transformed whole, both axes in one pass. Each lowering
 // can be named (EXPLICIT) where its kernels cover the shape.
@@ -380,17 +380,16 @@ class CompositeExecutor final : public Executor {
         std::vector<std::string> names;
         // A rank-2 FFT named explicitly as one of its lowerings takes that one
         // (EXPLICIT). Static rule: whole blocks in one pass where they fit; else
-        // axis 0 as column passes from 2^11-point axes, and from 2^9-point axes
-        // in 2^21 points or more; else transposing rows where their kernels cover
+        // axis 0 as column passes where an axis has 2^11 points, or axis 0 2^9 and
+        // the whole 2^21 or more; else transposing rows where their kernels cover
         // the shape, else transposes. Measured, us, transposes or transposing rows
         // / columns / blocks:
         //   32 x 32 (2^23 points) 199 / - / 30, (2^18) 25.9 / - / 6.9;
         //   128 x 64 124 / - / 33; 128 x 128 49.5 / 50.2 / 37.1;
-        //   256 x 256 47.4 / 48.3; 512 x 1024 66.7 / 54.9, (2^21) 27.1 / 23.2;
+        //   256 x 256 47.4 / 48.3; 256 x 1024 47.4 / 51.5;
+        //   512 x 1024 59.3 / 50.0, (2^21) 21.2 / 19.8, (2^19) 14.6 / 13.5;
         //   2048 x 2048 67.8 / 53.5.
-        // (Columns are as far ahead below 2^21 points: 512 x 1024, 2^19 points,
-        // 22.4 / 17.6. There the rows stay the default, which programs name, and
-        // the columns are MEASURE's choice.)
+        // (Below 2^21 points the two are close and the rows stay the default.)
         const bool named = r.policy == CUBUTTERFLY_ALGORITHM_EXPLICIT;
         const auto names_it = [&](const char* prefix) { return named && r.explicit_algorithm.rfind(prefix, 0) == 0; };
         const bool want_columns = force == 1 || names_it("rank2-columns[");
@@ -407,7 +406,7 @@ class CompositeExecutor final : public Executor {
             }
         }
         if (fft2 && !blocks_ && !want_rows &&
-            (want_columns || longest >= 11 || (longest >= 9 && r.n * r.batch >= (std::uint64_t{1} << 21)))) {
+            (want_columns || longest >= 11 || (logs[0] >= 9 && r.n * r.batch >= (std::uint64_t{1} << 21)))) {
             // Axis 0 as column passes over each block, then the rows.
             auto cols = make_fft_rank2_columns(axis_request(r.n, r.batch), logs[0]);
             if (cols) {

@@ -980,8 +980,25 @@ void add() {
 // transposing store with single-element segments.
 constexpr int single_li(int m) { return m < 12 ? 12 - m : 0; }
 constexpr int split_l1(int m) { return m / 2; }
-constexpr int col_lines(int l1, int l2) { return 14 - l1 < l2 ? 14 - l1 : l2; }
-constexpr int row_lines(int l1, int l2) { return 14 - l2 < l1 ? 14 - l2 : l1; }
+// Passes of 9 and more bits have three digits and no prefetching walk (one tile per
+// workgroup). Where the halved segments of 2^13-point tiles still pay, they take
+// those, two workgroups per CU, so that one loads while the other computes: column
+// passes of 9 bits (128-byte segments), row passes of 9 and 10 (128 and 64 bytes
+// transposed). 2^14- / 2^13-point tiles, us: 2^17 x 64 68.1 / 62.5, 2^18 x 4 24.5 /
+// 16.4, x 64 126 / 105, 2^19 x 32 128 / 111, 2^20 x 16 134 / 131. Column passes of 10
+// bits (64-byte segments) take them only where their 2^14-point tiles would leave
+// CUs idle (column_lines_for: 2^20 x 1 21.8 / 18.2, 2^21 x 1 30.8 / 27.7, but 2^21 x 4
+// 70.0 / 71.7).
+constexpr int col_lines(int l1, int l2) {
+    const int lines = l1 == 9 ? 13 - l1 : 14 - l1;
+    return lines < l2 ? lines : l2;
+}
+constexpr int row_lines(int l1, int l2) {
+    const int lines = l2 == 9 || l2 == 10 ? 13 - l2 : 14 - l2;
+    return lines < l1 ? lines : l1;
+}
+// The first column pass of a rank-2 block, its rows whole: 10 bits too.
+constexpr int rank2_column_lines(int ta) { return ta == 9 || ta == 10 ? 13 - ta : 14 - ta; }
 template <int M>
 void add_two() {
     constexpr int l1 = split_l1(M), l2 = M - l1;
@@ -992,10 +1009,14 @@ void add_two() {
 // Row passes over natural-order rows with the transposing store, tiles of
 // 2^14 points (2^(14 - LT) rows, at least 4 so the transposed segments are
 // 32 bytes or longer).
+// Rank-2 row passes with a transposing store: likewise (512 x 512 blocks, 2^19
+// points, both passes 22.2 / 14.6 us, 2^23 65.8 / 57.0).
+constexpr int transposed_lines(int l2) { return l2 == 9 || l2 == 10 ? 13 - l2 : 14 - l2; }
 template <int LT>
 void add_rows_natural() {
-    registry()[Key{LT, 14 - LT, false, false, false, 4}] = &launch<LT, 14 - LT, false, false, false, 4>;
-    registry()[Key{LT, 14 - LT, false, false, true, 4}] = &launch<LT, 14 - LT, false, false, true, 4>;
+    constexpr int li = transposed_lines(LT);
+    registry()[Key{LT, li, false, false, false, 4}] = &launch<LT, li, false, false, false, 4>;
+    registry()[Key{LT, li, false, false, true, 4}] = &launch<LT, li, false, false, true, 4>;
 }
 
 // Rank-2 blocks: column passes of 2^LT points over whole 2^14-point tiles,
@@ -1051,6 +1072,7 @@ void register_all() {
     add<4, 10, true, false>();
     add<5, 9, true, false>();
     add<6, 8, true, false>();
+    add<10, 3, true, false>();
     add_rank2_rows<5>();
     add_rank2_rows<6>();
     add_rank2_rows<7>();
@@ -1072,6 +1094,12 @@ Launch find(const Key& k) {
     const Launch fn = lookup(k);
     if (fn == nullptr) throw NotSupported("FFT pass shape has no gfx950 kernel");
     return fn;
+}
+
+// Column lines of a 1-D column pass over `points` points in all.
+int column_lines_for(int l1, int l2, std::uint64_t points) {
+    if (l1 == 10 && l2 >= 4 && (points >> 14) < std::uint64_t(device_cu_count())) return 3;
+    return col_lines(l1, l2);
 }
 
 // The final row pass's order flag: 32 for a bit-reversed output order.
@@ -1237,7 +1265,7 @@ class FftExecutor final : public Executor {
             algorithm = m >= 13 && !radix16 ? "fft-c64-resident-r32" : "fft-c64-resident-r16";
         } else {
             const std::uint32_t l1 = std::uint32_t(split), l2 = m - l1;
-            const int col_li = col_lines(int(l1), int(l2));
+            const int col_li = column_lines_for(int(l1), int(l2), r.batch << m);
             const int row_li = row_lines(int(l1), int(l2));
             const std::uint64_t col_tiles = r.batch << (l2 - col_li);
             const std::uint64_t row_tiles = r.batch << (l1 - row_li);
@@ -1368,7 +1396,7 @@ class FftRowsTransposedExecutor final : public Executor {
   public:
     FftRowsTransposedExecutor(const Request& r, std::uint32_t l1, Launch fn) : fn_(fn) {
         const std::uint32_t l2 = r.log_n;
-        const int li = 14 - int(l2);
+        const int li = transposed_lines(int(l2));
         // The row kernel forms level twiddles as powers of the 2^(l1 + l2)-th
         // root (w^(j << (m - h)) = the 2^h-th root's j-th power).
         upload_twiddles(twa_, twb_, int(l1 + l2), r.inverse);
@@ -1589,7 +1617,7 @@ class FftRank2ColumnsExecutor final : public Executor {
         // First column pass: the top ta bits of axis 0, columns = the rest of
         // the block (tb axis-0 bits, then l1 bits that are not transformed).
         {
-            const int li = 14 - int(ta);
+            const int li = rank2_column_lines(int(ta));
             Step s{find(Key{int(ta), li, true, false, r.inverse}), base, false, true};
             s.args.l1 = ta;
             s.args.l2 = tb + l1;
@@ -1681,13 +1709,13 @@ bool fft_rows_transposed_available(const Request& r, std::uint32_t l1) {
     // keeps a block's byte offsets in 32 bits).
     return l2 >= 4 && l2 <= 12 && int(l1) >= 14 - l2 && l1 + std::uint32_t(l2) <= 24 &&
            (r.batch & ((std::uint64_t{1} << l1) - 1)) == 0 &&
-           lookup(Key{l2, 14 - l2, false, false, r.inverse, 4}) != nullptr;
+           lookup(Key{l2, transposed_lines(l2), false, false, r.inverse, 4}) != nullptr;
 }
 
 std::unique_ptr<Executor> make_fft_rows_transposed(const Request& r, std::uint32_t l1) {
     if (!fft_rows_transposed_available(r, l1)) return nullptr;
     const int l2 = int(r.log_n);
-    return std::make_unique<FftRowsTransposedExecutor>(r, l1, lookup(Key{l2, 14 - l2, false, false, r.inverse, 4}));
+    return std::make_unique<FftRowsTransposedExecutor>(r, l1, lookup(Key{l2, transposed_lines(l2), false, false, r.inverse, 4}));
 }
 
 // The column-pass split of axis 0 (ta top bits, then tb; tb = 0 for one

@@ -83,8 +83,30 @@ def test_single_column_pass(torch_gpu, lib, stream, l0, l1, inverse):
         assert plan.mapping()["schedule"][0]["child"]["column_passes"] == 1
 
 
-@pytest.mark.parametrize("extents,batch,columns", [((512, 1024), 3, False), ((512, 1024), 4, True), ((256, 512), 16, True),
-                                                   ((256, 256), 64, False)])
+@pytest.mark.parametrize("extents,batch,columns", [((512, 1024), 3, False), ((512, 1024), 4, True), ((512, 256), 16, True),
+                                                   ((256, 512), 64, False), ((256, 256), 64, False)])
 def test_default_rule(torch_gpu, lib, extents, batch, columns):
     with cb.Plan(lib, fft_t(extents, batch)) as plan:
         assert plan.algorithm_name().startswith("rank2-columns[" if columns else "rank2-transposing[")
+
+
+# Two-pass 1-D lengths whose passes take halved tiles: 9-bit columns and 9- and
+# 10-bit rows always, 10-bit columns while their tiles are fewer than the CUs.
+@pytest.mark.parametrize("log_n,batch", [(17, 3), (18, 1), (18, 5), (19, 3), (20, 1), (20, 5), (21, 1), (21, 3)])
+@pytest.mark.parametrize("inverse", [False, True])
+def test_two_pass_tiles(torch_gpu, lib, stream, log_n, batch, inverse):
+    rng = np.random.default_rng(log_n + batch)
+    n = 1 << log_n
+    x = (rng.standard_normal((batch, n)) + 1j * rng.standard_normal((batch, n))).astype(np.complex64)
+    for orders in ([cb.LogicalOrder.NATURAL], [cb.LogicalOrder.BIT_REVERSED]):
+        t = cb.describe(cb.Operator.FFT, cb.DataType.COMPLEX_FP32, [n], batch, compute=cb.ComputeType.FP32,
+                        inverse=inverse, output_orders=orders)
+        got = run_plan(torch_gpu, lib, t, x, stream).astype(np.complex128)
+        ref = (np.fft.ifft if inverse else np.fft.fft)(x.astype(np.complex128), axis=1)
+        if orders[0] == cb.LogicalOrder.BIT_REVERSED:
+            perm = np.zeros(n, np.int64)
+            for b in range(log_n):
+                perm |= ((np.arange(n) >> b) & 1) << (log_n - 1 - b)
+            ref = ref[:, perm]
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert err <= 1e-6, err
