@@ -973,7 +973,8 @@ void add() {
 }
 
 // Shapes: one pass for m <= 14 (2^12-point tiles, 2^13 / 2^14 for m = 13,
-// 14); two passes with 2^14-point tiles over l1 = m / 2 high bits (column
+// 14); two passes with 2^14-point tiles (2^13 for some 9- and 10-bit passes,
+// below) over l1 = m / 2 high bits (column
 // tiles) and l2 = m - l1 low bits (row tiles). The even split keeps both the
 // column reads and the transposing row stores in segments of 2^(14 - m/2)
 // elements (32 bytes at m = 24); a column-heavier split would leave the
@@ -1722,9 +1723,9 @@ std::unique_ptr<Executor> make_fft_rows_transposed(const Request& r, std::uint32
 // pass), or false where no kernels cover the shape: rows of 2^5 .. 2^12
 // points (whole 2^14-point column tiles within a block), blocks of at most 2^24
 // points (the level-twiddle tables' reach), and axis 0 in one column pass of
-// 4 .. 11 bits, its 2^(14 - ta) columns within the 2^l1 of a row, or two: the
+// 4 .. 11 bits, its tile's columns within the 2^l1 of a row, or two: the
 // second over tb >= 14 - l1 bits, the first over the rest, each within 4 .. 8
-// bits. One pass of 9 to 11 bits moves segments of 256 to 64 bytes and still
+// bits. One pass of 9 to 11 bits moves segments of 128 or 64 bytes and still
 // beats two (2^23 points, 2048 x 1024: 53.8 against 74.7 us, 2048 x 2048 53.5
 // against 76.1). Blocks with 2^12-point rows keep two from 2^9 points on,
 // though one is faster there too (512 x 4096 x 2 50.4 / 33.3 us, 2048 x 4096 78.0
