@@ -581,7 +581,11 @@ class CompositeExecutor final : public Executor {
 
     // Ping-pong buffers of the packed data the schedule touches (0, 1 or 2):
     // the gather's target, then every step's destination but a direct last one.
+    // A column plan between a gather and a scatter runs in place on one buffer
+    // (its first pass leaves for the child's own workspace): two packed copies in
+    // all, as the transposing rows need there.
     std::size_t buffers() const {
+        if (in_place_child()) return 1;
         std::size_t used = direct_in_ ? 0 : 1;
         int next = direct_in_ ? 0 : 1;
         for (std::size_t i = 0; i < steps_.size(); ++i) {
@@ -592,6 +596,8 @@ class CompositeExecutor final : public Executor {
         }
         return used;
     }
+
+    bool in_place_child() const { return columns_ && !direct_in_ && !direct_out_; }
 
     // The last step that writes a new buffer (the in-place column passes
     // after it run on its destination).
@@ -657,7 +663,7 @@ class CompositeExecutor final : public Executor {
                                     narrow_here ? narrow : nullptr, out_scale);
                 continue;
             }
-            void* dst = i == last && direct_out_ ? out : buffer[next];
+            void* dst = in_place_child() ? buffer[0] : i == last && direct_out_ ? out : buffer[next];
             if (s.transpose) transpose(cur, dst, s, stream);
             else children_[s.child]->execute(cur, dst, child_ws, stream);
             cur = cur_writable = dst;
