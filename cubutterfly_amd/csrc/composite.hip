@@ -368,7 +368,8 @@ class CompositeExecutor final : public Executor {
   public:
     // force: 0 the static rule (or the name an EXPLICIT request gives), 1 a
     // rank-2 FFT's column passes, 2 its transposing row passes, 3 its one-pass
-    // blocks, 4 the static rule without them.
+    // blocks, 4 the static rule without them and without columns in place of
+    // transposes.
     CompositeExecutor(const Request& r, bool flatten, Selection* sel, int force = 0) : r_(r) {
         const std::uint32_t rank = r.rank;
         std::vector<std::uint32_t> logs(rank);
@@ -390,6 +391,12 @@ class CompositeExecutor final : public Executor {
         //   512 x 1024 59.3 / 50.0, (2^21) 21.2 / 19.8, (2^19) 14.6 / 13.5;
         //   2048 x 2048 67.8 / 53.5.
         // (Below 2^21 points the two are close and the rows stay the default.)
+        // Axis 0 beyond 2^11 points takes two column passes, and over rows of 2^6
+        // or 2^7 points those are slower than the transposing rows (4096 x 64,
+        // 2^18 points 21.6 / 25.4, 2^25 249 / 346; 4096 x 128, 2^19 23.3 / 30.3),
+        // which end at 2^12 points, and faster than the transposes beyond
+        // (8192 x 64, 2^19 30.1 / 27.7, 2^25 460 / 300), whose name stays a
+        // lowering of those shapes.
         const bool named = r.policy == CUBUTTERFLY_ALGORITHM_EXPLICIT;
         const auto names_it = [&](const char* prefix) { return named && r.explicit_algorithm.rfind(prefix, 0) == 0; };
         const bool want_columns = force == 1 || names_it("rank2-columns[");
@@ -405,30 +412,34 @@ class CompositeExecutor final : public Executor {
                 steps_.push_back(Step{false, 0, 0, 0, 0, 0});
             }
         }
-        if (fft2 && !blocks_ && !want_rows &&
-            (want_columns || longest >= 11 || (logs[0] >= 9 && r.n * r.batch >= (std::uint64_t{1} << 21)))) {
-            // Axis 0 as column passes over each block, then the rows.
+        // Axis 0 as column passes over each block, then the rows.
+        const auto try_columns = [&] {
             auto cols = make_fft_rank2_columns(axis_request(r.n, r.batch), logs[0]);
-            if (cols) {
-                columns_ = true;
-                children_.push_back(std::move(cols));
-                steps_.push_back(Step{false, 0, 0, 0, 0, 0});
-            }
-        }
-        if (fft2 && !blocks_ && !columns_ && !want_columns) {
-            // Each axis as one row pass that stores its blocks transposed:
-            // rows of the caller's layout, then rows of the transposed one,
-            // which lands back in the original order. No transpose kernels.
+            if (!cols) return;
+            columns_ = true;
+            children_.push_back(std::move(cols));
+            steps_.push_back(Step{false, 0, 0, 0, 0, 0});
+        };
+        // Each axis as one row pass that stores its blocks transposed: rows of
+        // the caller's layout, then rows of the transposed one, which lands back
+        // in the original order. No transpose kernels.
+        const auto try_rows = [&] {
             const std::uint64_t n0 = r.extents[0], n1 = r.extents[1];
             auto rows1 = make_fft_rows_transposed(axis_request(n1, r.batch * n0), logs[0]);
             auto rows0 = make_fft_rows_transposed(axis_request(n0, r.batch * n1), logs[1]);
-            if (rows1 && rows0) {
-                transposing_ = true;
-                children_.push_back(std::move(rows1));
-                children_.push_back(std::move(rows0));
-                steps_.push_back(Step{false, 0, 1, 0, 0, 0});
-                steps_.push_back(Step{false, 1, 0, 0, 0, 0});
-            }
+            if (!rows1 || !rows0) return;
+            transposing_ = true;
+            children_.push_back(std::move(rows1));
+            children_.push_back(std::move(rows0));
+            steps_.push_back(Step{false, 0, 1, 0, 0, 0});
+            steps_.push_back(Step{false, 1, 0, 0, 0, 0});
+        };
+        if (fft2 && !blocks_) {
+            const bool columns_rule = longest >= 11 || (logs[0] >= 9 && r.n * r.batch >= (std::uint64_t{1} << 21));
+            const bool rows_first = two_column_passes_over_short_rows(logs);
+            if (want_columns || (!want_rows && columns_rule && !rows_first)) try_columns();
+            if (!columns_ && !want_columns) try_rows();
+            if (rows_first && !transposing_ && !named && force == 0) try_columns();
         }
         if (transposing_ || columns_ || blocks_) {
         } else if (flatten) {
@@ -680,12 +691,23 @@ class CompositeExecutor final : public Executor {
                fft_rows_transposed_available(axis_request_of(r, r.extents[0], r.batch * r.extents[1]), l1);
     }
 
+    // Whether its default is column passes where the other lowering is
+    // transposes that would measure their axes' plans (no device work).
+    static bool columns_over_transposes(const Request& r) {
+        return two_column_passes_over_short_rows({log2_u64(r.extents[0]), log2_u64(r.extents[1])}) &&
+               fft_rank2_columns_available(axis_request_of(r, r.n, r.batch), log2_u64(r.extents[0])) &&
+               !both_rank2_lowerings(r);
+    }
+
     // Whether it has the one-pass blocks (no device work).
     static bool fits_blocks(const Request& r) {
         return fft_rank2_blocks_available(axis_request_of(r, r.n, r.batch), log2_u64(r.extents[0]));
     }
 
   private:
+    static bool two_column_passes_over_short_rows(const std::vector<std::uint32_t>& logs) {
+        return logs[0] > 11 && logs[1] < 8;
+    }
     Request axis_request(std::uint64_t n, std::uint64_t batch) const { return axis_request_of(r_, n, batch); }
     static Request axis_request_of(const Request& r, std::uint64_t n, std::uint64_t batch) {
         Request c = r;
@@ -952,7 +974,8 @@ std::unique_ptr<Executor> make_composite_executor(const Request& r, Selection* s
             }
         } else {
             const bool both = CompositeExecutor::both_rank2_lowerings(r), whole = CompositeExecutor::fits_blocks(r);
-            if (both || whole) {
+            const bool long_columns = CompositeExecutor::columns_over_transposes(r);
+            if (both || whole || long_columns) {
                 require_no_capture(*sel);
                 std::vector<std::unique_ptr<Executor>> alternatives;
                 const auto offer = [&](int force, bool (CompositeExecutor::*is)() const) {
@@ -963,6 +986,7 @@ std::unique_ptr<Executor> make_composite_executor(const Request& r, Selection* s
                     offer(1, &CompositeExecutor::columns);
                     offer(2, &CompositeExecutor::transposing);
                 } else {
+                    if (long_columns) offer(1, &CompositeExecutor::columns);
                     offer(4, nullptr);
                 }
                 if (whole) offer(3, &CompositeExecutor::blocks);
