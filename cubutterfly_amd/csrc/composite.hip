@@ -17,7 +17,8 @@
 // The transposing store writes segments of 2^(14 - n) elements for rows of
 // 2^n points; where an axis has 2^11 points or more (segments under 128
 // bytes), or axis 0 2^9 in 2^21 points or more, the block runs instead as column
-// passes over axis 0 and a row pass over axis 1 that stores whole rows. Blocks of
+// passes over axis 0 and a row pass over axis 1 that stores whole rows (the
+// exceptions stand at the rule in CompositeExecutor). Blocks of
 // at most 2^14 points are transformed whole, both axes in one pass. Each lowering
 // can be named (EXPLICIT) where its kernels cover the shape.
 //
@@ -390,7 +391,13 @@ class CompositeExecutor final : public Executor {
         //   256 x 256 47.4 / 48.3; 256 x 1024 47.4 / 51.5;
         //   512 x 1024 59.3 / 50.0, (2^21) 21.2 / 19.8, (2^19) 14.6 / 13.5;
         //   2048 x 2048 67.8 / 53.5.
-        // (Below 2^21 points the two are close and the rows stay the default.)
+        // (Below 2^21 points the two are close and the rows stay the default.) One
+        // column pass of 9 to 11 bits writes segments of 64 or 128 bytes, which cost
+        // more once nothing stays in the Infinity Cache: from 2^25 points the rows
+        // are faster again where axis 1 is short (us at 2^24 / 2^25 / 2^26, rows
+        // then columns: 512 x 256 110, 93 / 214, 216 / 396, 436; 1024 x 512 98, 101 /
+        // 227, 237 / 423, 432; 2048 x 32 132, 112 / 250, 261 / 470, 528; 512 x 1024
+        // 98, 105 / 226, 246 / 423, 440; but 1024 x 1024 115, 114 / 294, 269 / 568, 501).
         // Axis 0 beyond 2^11 points takes two column passes, and over rows of 2^6
         // or 2^7 points those are slower than the transposing rows (4096 x 64,
         // 2^18 points 21.6 / 25.4, 2^25 249 / 346; 4096 x 128, 2^19 23.3 / 30.3),
@@ -436,7 +443,9 @@ class CompositeExecutor final : public Executor {
         };
         if (fft2 && !blocks_) {
             const bool columns_rule = longest >= 11 || (logs[0] >= 9 && r.n * r.batch >= (std::uint64_t{1} << 21));
-            const bool rows_first = two_column_passes_over_short_rows(logs);
+            const bool large = r.n * r.batch >= (std::uint64_t{1} << 25);
+            const bool rows_first = two_column_passes_over_short_rows(logs) ||
+                                    (large && logs[0] >= 9 && logs[0] <= 11 && logs[1] <= (logs[0] == 9 ? 10u : 9u));
             if (want_columns || (!want_rows && columns_rule && !rows_first)) try_columns();
             if (!columns_ && !want_columns) try_rows();
             if (rows_first && !transposing_ && !named && force == 0) try_columns();

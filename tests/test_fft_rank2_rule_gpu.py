@@ -37,6 +37,16 @@ def test_short_rows(torch_gpu, lib, stream, l0, l1, prefix, inverse):
     check(torch_gpu, lib, stream, (1 << l0, 1 << l1), 2 if l0 < 13 else 1, prefix, inverse=inverse)
 
 
+# One column pass of 9 to 11 bits over short rows: up to 2^24 points in all.
+@pytest.mark.parametrize("extents,batch,prefix", [
+    ((2048, 32), 256, COLUMNS), ((2048, 32), 512, ROWS), ((512, 256), 255, COLUMNS), ((512, 256), 256, ROWS),
+    ((2048, 512), 32, ROWS), ((1024, 512), 63, COLUMNS), ((1024, 512), 64, ROWS), ((512, 1024), 64, ROWS),
+    ((1024, 1024), 32, COLUMNS), ((256, 2048), 64, COLUMNS), ((512, 2048), 32, COLUMNS)])
+def test_large_batches(torch_gpu, lib, extents, batch, prefix):
+    with cb.Plan(lib, fft_t(extents, batch)) as plan:
+        assert plan.algorithm_name().startswith(prefix)
+
+
 def transposes(l0, l1):
     leaf = {6: "resident-r16", 7: "resident-r16", 13: "resident-r32", 15: "two-pass-r16"}
     return f"{TRANSPOSES}fft-c64-{leaf[l1]},fft-c64-{leaf[l0]}]+direct-input+direct-output"
