@@ -1074,6 +1074,8 @@ void register_all() {
     add<5, 9, true, false>();
     add<6, 8, true, false>();
     add<10, 3, true, false>();
+    registry()[Key{10, 4, false, false, false}] = &launch<10, 4, false, false, false, 0>;
+    registry()[Key{10, 4, false, false, true}] = &launch<10, 4, false, false, true, 0>;
     add_rank2_rows<5>();
     add_rank2_rows<6>();
     add_rank2_rows<7>();
@@ -1101,6 +1103,17 @@ Launch find(const Key& k) {
 int column_lines_for(int l1, int l2, std::uint64_t points) {
     if (l1 == 10 && l2 >= 4 && (points >> 14) < std::uint64_t(device_cu_count())) return 3;
     return col_lines(l1, l2);
+}
+
+// Row lines of a 1-D final row pass over `points` points in all: the 64-byte
+// transposed segments of 2^13-point tiles of 10-bit rows cost more than they gain
+// once nothing stays in the Infinity Cache (2^20 natural order, 2^14- / 2^13-point
+// tiles: x 8 67.4 / 62.3 us, x 32 307.1 / 313.1, x 64 inverse 556.0 / 580.1; the
+// bit-reversed order, which stores whole rows, gains at every size). 9-bit columns
+// before it (2^19) keep the two level from 2^25 points on.
+int row_lines_for(int l1, int l2, std::uint64_t points, int ord) {
+    if (l1 == 10 && l2 == 10 && ord == 0 && points >= (std::uint64_t{1} << 25)) return 4;
+    return row_lines(l1, l2);
 }
 
 // The final row pass's order flag: 32 for a bit-reversed output order.
@@ -1211,6 +1224,7 @@ class FftExecutor final : public Executor {
         base.scale = scale;
         const std::uint64_t in_pitch = r.pitched ? r.in_batch_stride : r.n;
         const std::uint64_t out_pitch = r.pitched ? r.out_batch_stride : r.n;
+        unsigned row_tile_lines = 0;  // two-pass plans
         if (mid > 0) {
             const std::uint32_t ta = std::uint32_t(split), tm = std::uint32_t(mid), tl = m - ta - tm;
             upload_twiddles(sub_twa_, sub_twb_, int(tm + tl), r.inverse);
@@ -1267,7 +1281,7 @@ class FftExecutor final : public Executor {
         } else {
             const std::uint32_t l1 = std::uint32_t(split), l2 = m - l1;
             const int col_li = column_lines_for(int(l1), int(l2), r.batch << m);
-            const int row_li = row_lines(int(l1), int(l2));
+            const int row_li = row_lines_for(int(l1), int(l2), r.batch << m, row_ord(r));
             const std::uint64_t col_tiles = r.batch << (l2 - col_li);
             const std::uint64_t row_tiles = r.batch << (l1 - row_li);
             require(col_tiles <= 0xffffffffull && row_tiles <= 0xffffffffull, "FFT batch exceeds the grid");
@@ -1289,6 +1303,7 @@ class FftExecutor final : public Executor {
             steps_ = {a, b};
             workspace_ = static_cast<std::size_t>(r.batch << m) * sizeof(float2);
             algorithm = two_pass_name(int(m), int(l1));
+            row_tile_lines = 1u << row_li;
         }
         algorithm += order_suffix(r);
         if (r.pitched) algorithm += "-pitched";
@@ -1306,6 +1321,7 @@ class FftExecutor final : public Executor {
             .field("passes", unsigned(steps_.size()))
             .field("column_bits", unsigned(split))
             .field("middle_bits", unsigned(mid))
+            .field("row_tile_lines", row_tile_lines)
             .field("workspace_bytes", std::uint64_t(workspace_))
             .end_object();
         mapping_json = w.str();
