@@ -1045,8 +1045,19 @@ struct Pass {
     }
 };
 
+// Waves per SIMD that a pass kernel is compiled for: one workgroup's, but two
+// workgroups' for forward u64 rows of 2^13 points with both boundaries staged. Those
+// took 131 registers, which left one workgroup per CU where the LDS has room for two
+// (reused / rotated buffers: 512 rows 32.3 -> 27.1 us / 37.0 -> 29.3, 1025 rows
+// 68.1 -> 51.6 / 75.8 -> 57.1; up to 256 rows unchanged).
+template <class W, int LT, int LI, bool CT, bool PIN, bool POUT, bool SINGLE>
+constexpr int min_waves() {
+    return SINGLE && LT == 13 && sizeof(W) == 8 && CT && PIN && POUT ? 4 : imax((1 << (LT + LI - kLE)) / 256, 1);
+}
+
 template <class W, int AR, int LT, int LI, bool COL, bool CT, bool PIN, bool POUT, bool SINGLE, int L1, int L2>
-__global__ __launch_bounds__(1 << (LT + LI - kLE)) void ntt_pass_kernel(PassArgs<W> a) {
+__global__ __launch_bounds__(1 << (LT + LI - kLE), (min_waves<W, LT, LI, CT, PIN, POUT, SINGLE>())) void ntt_pass_kernel(
+    PassArgs<W> a) {
     Pass<W, AR, LT, LI, COL, CT, PIN, POUT, SINGLE, L1, L2>::run(a);
 }
 
