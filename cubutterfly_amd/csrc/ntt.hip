@@ -140,9 +140,7 @@ struct EngineImplT {
         lazy = !c.force_strict && !c.barrett && max_q < (std::uint64_t{1} << (bits - 2));
         supported(!c.barrett || max_q < (std::uint64_t{1} << (bits - 2)),
                   "Barrett arithmetic needs every modulus below 2^" + std::to_string(bits - 2));
-        // Moduli that leave four spare bits (and whose reciprocal fits 32) take
-        // the headroom form of the lazy butterflies.
-        const bool headroom = lazy && bits == 64 && max_q < (std::uint64_t{1} << 60) && min_q >= (std::uint64_t{1} << 33);
+        const bool headroom = lazy && ntt_headroom(bits, min_q, max_q);
         arith = c.barrett ? kBarrett : headroom ? kHeadroom : lazy ? kLazy : kStrict;
         const std::uint64_t polys = c.polynomials.empty() ? c.batch : c.polynomials.size();
         require(polys >= 1 && polys <= 0xffffffffull, "NTT batch must be in [1, 2^32)");
@@ -403,30 +401,64 @@ std::vector<std::uint32_t> ntt_other_splits(std::uint32_t log_n) {
     return out;
 }
 
+bool ntt_headroom(std::uint32_t word_bits, std::uint64_t min_q, std::uint64_t max_q) {
+    return word_bits == 64 && max_q < (std::uint64_t{1} << 60) && min_q >= (std::uint64_t{1} << 33);
+}
+
 // Whole 2^13- / 2^14-point polynomials in one workgroup each: one round trip
-// through memory and one launch in place of two, but a batch has to fill the
-// chip. Measured with both lowerings over 5 .. 1024 polynomials, back-to-back
-// calls (two passes / resident, us, forward in native order):
-//   u32 2^13: 8 8.1 / 6.1, 64 8.1 / 6.3, 512 15.2 / 12.0, 1024 26.9 / 19.5
-//   u32 2^14: 64 8.1 / 9.9, 128 10.9 / 10.8, 192 13.5 / 11.8, 1024 57.7 / 45.3
-//   u64 2^13: 64 11.5 / 12.6, 128 13.5 / 13.4, 256 17.8 / 15.8, 1024 71 / 50
-//   u64 2^14: 64 15.5 / 22.5, 192 26.4 / 25.8, 256 36.4 / 27.8, 257 37.5 / 45.1,
-//             512 75 / 59
-// The other direction and orders cross at the same counts. A request is
-// offered the lowering (MEASURE, RNS Prepare) from about half of where it starts
-// to win; 2^13-point u32 rows from one per XCD.
+// through memory and one launch in place of two. A request is offered the lowering
+// (MEASURE, RNS Prepare) from about half of where it starts to win; 2^13-point u32
+// rows from one per XCD.
 bool ntt_resident_offered(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys, bool barrett) {
     if (barrett || (log_n != 13 && log_n != 14)) return false;
     return polys >= (word_bits == 64 ? 96u : log_n == 14 ? 64u : 8u);
 }
 
-bool ntt_resident_default(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys) {
-    if (!ntt_resident_offered(word_bits, log_n, polys, false)) return false;
+// The rows are bound by arithmetic, so a batch takes as long as its fullest CU: it
+// runs in rounds of one row per CU, and the two passes are faster where the last
+// round is far from full. Resident over two-pass time in graph replays, on reused /
+// rotated buffers, directions and orders as ranges (256 CUs):
+//   u64 2^13: 130 rows 0.77-0.86 / 0.76-0.86, 256 0.81-0.92 / 0.81-0.93; 300
+//             1.05-1.14 / 1.01-1.12, 360 1.02-1.11 / 0.97-1.12, 400 0.87-0.98 /
+//             0.83-0.92, 512 0.82-0.95 / 0.79-0.90; with headroom 540 1.00-1.08 /
+//             0.92-0.98, 680 0.87-0.93 / 0.83-0.91, 1100 0.97-1.03 / 0.90-0.96;
+//             without 540 1.07-1.14 / 0.95-1.07, 680 0.93-1.02 / 0.87-0.98, 1100
+//             1.03-1.10 / 0.93-1.06
+//   u64 2^14: 190 0.97-1.17 / 0.94-1.14, 205 0.89-1.06 / 0.84-1.01, 256 0.88-1.06 /
+//             0.78-0.99; 410 1.10-1.38 / 1.03-1.30, 512 0.99-1.20 / 0.86-1.10, 1024
+//             0.94-1.22 / 1.00-1.29 (139 KB of LDS: nothing overlaps a row's loads
+//             and stores)
+//   u32 2^14, no LDS permutation (forward to bit-reversed order, inverse from it):
+//             140 0.87-0.97 / 0.83-0.97, 256 0.71-0.83; 280 1.07 / 0.93-1.05, 330
+//             0.92-0.98 / 0.86-0.93, 512 0.73-0.83 / 0.68-0.79; 540 0.97-1.02 /
+//             0.88-0.91, 1025 0.92-1.00 / 0.81-0.89
+//   u32 2^14, others: 140 0.92-1.00, 256 0.75-0.86; 300 1.11-1.19 / 0.95-1.13, 360
+//             0.97-1.05 / 0.90-1.02, 400 0.92-0.99 / 0.82-0.94, 512 0.85-0.98 /
+//             0.76-0.89; 620 1.04-1.11 / 0.88-1.03, 700 0.98-1.06 / 0.81-0.96, 820
+//             1.10-1.17 / 0.94-1.09. Forward to natural order is at the upper ends
+//             (from 700 rows 1.05-1.14 / 0.94-1.11), and above them from
+//             bit-reversed input or with full reduction (160 1.06-1.07, 200
+//             0.90-0.95, 400 1.05-1.06 / 1.02-1.05, 700 1.13-1.15 / 1.04-1.12).
+// u32 2^13 rows win from 128 on everywhere (0.64-1.05). Below, a forward call takes
+// 6.4-7.1 us against 5.9-6.6 in a graph replay, and 6.1 against 8.1 where the host
+// issues each launch (8 rows): one launch, then, from 8 rows on.
+bool ntt_resident_default(const NttResidentUse& u) {
+    if (!ntt_resident_offered(u.word_bits, u.log_n, u.polys, false)) return false;
+    const bool u32 = u.word_bits == 32;
     const std::uint64_t cus = std::uint64_t(device_cu_count());
-    // u64 2^14-point rows take a CU's LDS each and run in rounds of one per CU:
-    // where the last round is not nearly full the two passes are faster.
-    if (word_bits == 64 && log_n == 14) return polys * 5 >= (polys + cus - 1) / cus * cus * 4;
-    return (word_bits == 32 && log_n == 13) || polys > cus / 2;
+    const std::uint64_t rounds = (u.polys + cus - 1) / cus;
+    const auto full = [&](unsigned num, unsigned den) { return u.polys * den >= rounds * cus * num; };  // num / den of it
+    if (u32 && u.log_n == 13) return true;
+    if (u.log_n == 13)
+        return rounds == 1 ? u.polys * 2 > cus : rounds == 2 ? full(3, 4) : u.headroom || full(7, 8);
+    if (!u32) return rounds == 1 && full(4, 5);
+    const bool to_natural = !u.inverse && !u.output_bit_reversed;
+    const bool unpermuted = u.inverse ? u.input_bit_reversed && !u.output_bit_reversed
+                                      : !u.input_bit_reversed && u.output_bit_reversed;
+    if (to_natural && (u.input_bit_reversed || u.strict)) return rounds == 1 && full(3, 4);
+    if (rounds == 1 || unpermuted) return u.polys * 2 > cus;
+    if (to_natural) return rounds == 2 && full(3, 4);
+    return rounds == 2 ? full(2, 3) : full(7, 8);
 }
 
 std::size_t NttEngine::workspace_bytes() const {
@@ -460,7 +492,11 @@ bool wide_columns_default(const Request& r) { return r.word_bits == 32 && r.log_
 
 std::vector<std::uint32_t> other_splits(const Request& r) { return ntt_other_splits(r.log_n); }
 
-bool resident_default(const Request& r) { return ntt_resident_default(r.word_bits, r.log_n, r.batch); }
+bool resident_default(const Request& r) {
+    return ntt_resident_default({r.word_bits, r.log_n, r.batch, r.inverse, r.input_bit_reversed, r.output_bit_reversed,
+                                 r.modulus >= (std::uint64_t{1} << (r.word_bits - 2)),
+                                 ntt_headroom(r.word_bits, r.modulus, r.modulus)});
+}
 
 std::string family_name(const Request& r) {
     return "ntt-u" + std::to_string(r.word_bits) + (r.negacyclic ? "-negacyclic" : "-cyclic");

@@ -11,10 +11,10 @@
 // times n^-1. Natural/bit-reversed boundaries are LDS-staged permutations of
 // the first or last pass.
 //
-// Lengths up to 2^12 (2^13 and 2^14 in batches that fill the chip) run in one
-// pass (whole polynomials resident in a workgroup); others in two passes over the high and low index bits,
-// each an in-register radix-16 / LDS-exchange core, with the intermediate in
-// a workspace of polys * n words.
+// Lengths up to 2^12 (2^13 and 2^14 where ntt_resident_default says so) run in
+// one pass (whole polynomials resident in a workgroup); others in two passes over
+// the high and low index bits, each an in-register radix-16 / LDS-exchange core,
+// with the intermediate in a workspace of polys * n words.
 #pragma once
 
 #include "common.hpp"
@@ -76,10 +76,21 @@ class NttEngine {
 // 2^log_n (the `-h<l1>` lowerings), empty elsewhere.
 std::vector<std::uint32_t> ntt_other_splits(std::uint32_t log_n);
 
+// Whether moduli in [min_q, max_q] leave four spare bits of a u64 word and have a
+// reciprocal of 32 bits: their lazy butterflies take the headroom form.
+bool ntt_headroom(std::uint32_t word_bits, std::uint64_t min_q, std::uint64_t max_q);
+
 // Whether 2^log_n-point polynomials may run whole in one workgroup each
 // (NttEngineConfig::resident) where `polys` of them run at once.
 bool ntt_resident_offered(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys, bool barrett);
 // Whether that is the static model's choice.
-bool ntt_resident_default(std::uint32_t word_bits, std::uint32_t log_n, std::uint64_t polys);
+struct NttResidentUse {
+    std::uint32_t word_bits, log_n;
+    std::uint64_t polys;
+    bool inverse, input_bit_reversed, output_bit_reversed;
+    bool strict;    // moduli of 2^(word bits - 2) and more
+    bool headroom;  // ntt_headroom
+};
+bool ntt_resident_default(const NttResidentUse& u);
 
 }  // namespace cbw

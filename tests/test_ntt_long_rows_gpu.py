@@ -84,14 +84,51 @@ def test_u64_moduli(torch_gpu, lib, stream, kind, log_n, inverse):
     check(torch_gpu, lib, stream, 64, log_n, 3, U64[kind], cb.NttRing.NEGACYCLIC, inverse, False, False)
 
 
+# (256 CUs) The edges of the rule, in natural order: a round half full (u64 2^14:
+# four fifths of one, and no more rounds), two rounds three quarters full; u64 2^13
+# any number of rounds beyond.
 @pytest.mark.parametrize("bits,log_n,batch,resident", [(32, 13, 4, False), (32, 13, 8, True), (32, 14, 128, False),
                                                        (32, 14, 129, True), (64, 13, 128, False), (64, 13, 129, True),
-                                                       (64, 14, 204, False), (64, 14, 205, True), (64, 14, 257, False),
-                                                       (64, 14, 410, True)])
+                                                       (64, 14, 204, False), (64, 14, 205, True), (64, 14, 256, True),
+                                                       (64, 14, 257, False), (64, 14, 410, False), (64, 14, 512, False),
+                                                       (64, 13, 257, False), (64, 13, 383, False), (64, 13, 384, True),
+                                                       (64, 13, 513, True), (32, 14, 300, False), (32, 14, 383, False),
+                                                       (32, 14, 384, True), (32, 14, 513, False)])
 def test_default_rule(torch_gpu, lib, bits, log_n, batch, resident):
-    q = U32["lazy"] if bits == 32 else U64["headroom-top"]
+    expect_resident(lib, bits, log_n, batch, resident)
+
+
+# More than two rounds of u64 2^13 without headroom: seven eighths full.
+@pytest.mark.parametrize("batch,resident", [(384, True), (513, False), (671, False), (672, True)])
+def test_default_rule_without_headroom(torch_gpu, lib, batch, resident):
+    for kind in ("lazy", "strict"):
+        expect_resident(lib, 64, 13, batch, resident, kind)
+
+
+# u32 2^14 by direction and order: forward to natural order from bit-reversed input,
+# or with full reduction, in the first round only; rows that need no permutation in
+# every round; the others two thirds of two rounds, seven eighths of more.
+@pytest.mark.parametrize("batch,inverse,rin,rout,strict,resident", [
+    (160, False, True, False, False, False), (192, False, True, False, False, True),
+    (512, False, True, False, False, False), (160, False, False, False, True, False),
+    (192, False, False, False, True, True), (512, False, False, False, True, False),
+    (257, False, False, True, True, True), (700, False, False, True, False, True),
+    (257, True, True, False, False, True), (128, True, True, False, False, False),
+    (341, True, False, False, False, False), (342, True, False, False, False, True),
+    (671, True, False, True, False, False), (672, True, False, True, False, True)])
+def test_default_rule_by_order(torch_gpu, lib, batch, inverse, rin, rout, strict, resident):
+    expect_resident(lib, 32, 14, batch, resident, "strict" if strict else "lazy", inverse=inverse, ntt_input_layout=LAYOUT[rin],
+                    ntt_output_layout=LAYOUT[rout])
+
+
+LAYOUT = {False: cb.NttLayout.NATURAL, True: cb.NttLayout.BIT_REVERSED}
+
+
+def expect_resident(lib, bits, log_n, batch, resident, kind=None, **fields):
+    q = U32[kind or "lazy"] if bits == 32 else U64[kind or "headroom-top"]
     t = cb.describe(cb.Operator.NTT, cb.DataType.UINT32 if bits == 32 else cb.DataType.UINT64, [1 << log_n], batch,
-                    compute=cb.ComputeType.UINT32 if bits == 32 else cb.ComputeType.UINT64, modulus=q, word_bits=bits)
+                    compute=cb.ComputeType.UINT32 if bits == 32 else cb.ComputeType.UINT64, modulus=q, word_bits=bits,
+                    **fields)
     with cb.Plan(lib, t) as plan:
         assert ("resident" in plan.algorithm_name()) == resident
         assert (plan.workspace_size() == 0) == resident
