@@ -514,13 +514,16 @@ struct Pass {
     // own rows, kStagedAux: C2 38.6 -> 37.3 us, C4 54.2 -> 52.0), and forward
     // column passes whose tiles write whole 128-byte lines per row (u32
     // 32-column, u64 16-column tiles), which the row pass then finds in the
-    // Infinity Cache where nontemporal stores left it to memory: forward and
-    // inverse of u32 2^16 x 64 36.3 -> 35.0 us, x 128 73.3 -> 65.9; u64 2^16 x 32
-    // 41.9 -> 41.1, x 64 76.1 -> 72.3. Forward column passes of narrower tiles keep
-    // write-back stores: write-through made them slower (partial-line segments
-    // that the L2 would otherwise merge). (Nontemporal final stores measured
-    // slower for C4, whose bit-reversed output lands in 8-byte segments: 60.6 ->
-    // 71-73 us.)
+    // Infinity Cache where nontemporal stores left it to memory. Forward and
+    // inverse, nontemporal / write-through, reused and rotated buffers: u32 2^16 x
+    // 64 34.9 / 35.0, 37.9 / 38.8; x 96 53.9 / 46.8, 59.2 / 51.7; x 256 120.6 /
+    // 107.3, 134.4 / 116.0; u64 2^16 x 64 72.6 / 72.8, 76.8 / 77.0; x 256 272.5 /
+    // 243.5, 274.2 / 245.1. Only intermediates of 8 MiB lose, in the forward call
+    // by itself (u32 2^16 x 32 10.2 / 10.7, u64 x 16 15.1 / 15.6; with the inverse
+    // after it within 1%). Forward column passes of narrower tiles keep write-back
+    // stores: write-through made them slower (partial-line segments that the L2
+    // would otherwise merge). (Nontemporal final stores measured slower for C4,
+    // whose bit-reversed output lands in 8-byte segments: 60.6 -> 71-73 us.)
     static constexpr int kStoreAux =
         !SINGLE && (!CT || (COL ? (sizeof(W) << LI) >= 128 : POUT)) ? 17 : 0;
     // A register window starting at tile bit S <= 6 leaves tile bits 10 and up
@@ -545,11 +548,15 @@ struct Pass {
     // wave's rows, measured no faster: C4 52.7 against 52.0-52.2 us.)
     static constexpr int kPer = 16 / int(sizeof(W));  // words per 16-byte access
     // Twiddle chunks one phase ahead: u32 two-pass tiles have the registers (95 of
-    // the 128 that 4 waves per SIMD allow, and a batch of 64 fills no more) and
-    // gain the L2 latency of each phase: u32 2^16 x 64 forward and inverse 35.3 ->
-    // 34.3 us, x 128 66.4 -> 63.3. u64 tiles lose occupancy for it (2^16 x 32 41.7 ->
-    // 43.3 us), and one-pass tiles run more waves per SIMD.
-    static constexpr bool kAhead = sizeof(W) == 4 && !SINGLE && !BARRETT && kPhases <= 3;
+    // the 128 that 4 waves per SIMD allow) and gain the L2 latency of each phase.
+    // Forward and inverse, us without / with it, reused and rotated buffers: 2^15 x
+    // 256 61.6 / 59.4, 75.2 / 70.1; 2^17 x 64 74.3 / 71.0, 86.7 / 81.8; below 2^23
+    // points level. The forward pass of 32-column tiles does without: 2^16 x 64 on
+    // rotated buffers 38.2 / 38.8 (x 56 37.3 / 38.0, x 40 32.0 / 32.5), other sizes
+    // and reused buffers within 1%. u64 tiles lose occupancy for it (2^16 x 32 41.7
+    // -> 43.3 us), and one-pass tiles run more waves per SIMD.
+    static constexpr bool kAhead = sizeof(W) == 4 && !SINGLE && !BARRETT && kPhases <= 3 &&
+                                   !(COL && CT && (sizeof(W) << LI) >= 128);
 
     // Staged store run: lane l of wave w moves tile elements g0 + 64 kPer k + e
     // (e < kPer), g0 = 1024 w + kPer l. The thread, lane and register parts
