@@ -26,6 +26,7 @@
 
 #include "buffer.hpp"
 #include "ntt_engine.hpp"
+#include "ntt_schedule.hpp"
 
 #include <cstddef>
 #include <map>
@@ -35,9 +36,6 @@
 
 namespace cbw {
 namespace ntt_detail {
-
-constexpr int kLE = 4;
-constexpr int kE = 1 << kLE;
 
 // A twiddle and its Shoup factor floor(w 2^k / q). Tables of lazy
 // Cooley-Tukey passes hold -w mod 2^k in place of w (see ct_butterfly).
@@ -86,71 +84,6 @@ struct PassArgs {
     std::uint32_t phase_off[4];  // chunk array of each phase, entries from the domain's table start
     std::uint32_t tw_bytes;      // bytes of one domain's chunk tables (buffer range of the twiddle reads)
 };
-
-// ---- phase geometry (host and device) ---------------------------------------
-//
-// A pass butterflies LT transform bits in phases of a 4-bit register window.
-// Cooley-Tukey (CT) walks the bits high -> low, windows [LT-4(P+1), LT-4P)
-// clamped at 0; Gentleman-Sande (GS) walks low -> high, windows [4P, 4P+4)
-// clamped at LT-4. A clamped window re-covers bits of its neighbour; only the
-// bits not yet done ("active" stages) are butterflied there. Whole rows of
-// 2^13 and 2^14 points (kLongRow) take the CT windows in reverse order for GS
-// as well, so the clamped window is the lowest one in both directions and all
-// exchanges but one stay inside a wave (Pass::wave_local).
-
-constexpr int num_phases(int lt) { return (lt + kLE - 1) / kLE; }
-constexpr int imin(int a, int b) { return a < b ? a : b; }
-constexpr int imax(int a, int b) { return a > b ? a : b; }
-
-constexpr int kLongRow = 13;  // one-pass rows from 2^13 points
-constexpr int window_start(int lt, bool ct, int p) {
-    if (!ct && lt >= kLongRow) return window_start(lt, true, num_phases(lt) - 1 - p);
-    return ct ? imax(lt - kLE * (p + 1), 0) : (kLE * p < lt - kLE ? kLE * p : imax(lt - kLE, 0));
-}
-constexpr int stage_hi(int lt, bool ct, int p) {
-    if (!ct && lt >= kLongRow) return stage_hi(lt, true, num_phases(lt) - 1 - p);
-    const int ws = window_start(lt, ct, p);
-    return ct ? imin(imin(ws + 3, lt - 1), lt - kLE * p - 1) : imin(ws + 3, lt - 1);
-}
-constexpr int stage_lo(int lt, bool ct, int p) {
-    if (!ct && lt >= kLongRow) return stage_lo(lt, true, num_phases(lt) - 1 - p);
-    const int ws = window_start(lt, ct, p);
-    return ct ? ws : imax(ws, kLE * p);
-}
-// Stage k of the phase at window ws: its twiddle for register group g is
-// table[(head >> (k+1)) + (g & gmask)], head = (prefix << lt) | (window bits
-// clear). Distinct entries per thread: 2^min(ws+3-k, lt-1-k). All of a
-// phase's entries hang off the block index head >> chunk_shift.
-constexpr int stage_count(int lt, int ws, int k) { return 1 << imin(ws + 3 - k, lt - 1 - k); }
-constexpr int chunk_shift(int lt, bool ct, int p) { return imin(window_start(lt, ct, p) + kLE, lt); }
-// The final GS stage of a transform multiplies by n^-1 (no table entries).
-constexpr bool scale_stage(int lt, bool ct, bool last, int k) { return !ct && last && k == lt - 1; }
-// k of the s-th executed stage of a phase.
-constexpr int exec_stage(int lt, bool ct, int p, int s) { return ct ? stage_hi(lt, ct, p) - s : stage_lo(lt, ct, p) + s; }
-constexpr int active_stages(int lt, bool ct, int p) { return stage_hi(lt, ct, p) - stage_lo(lt, ct, p) + 1; }
-// Entry offset of the s-th executed stage within the chunk, and the chunk size.
-constexpr int chunk_offset(int lt, bool ct, bool last, int p, int s) {
-    int off = 0;
-    for (int e = 0; e < s; ++e) {
-        const int k = exec_stage(lt, ct, p, e);
-        if (!scale_stage(lt, ct, last, k)) off += stage_count(lt, window_start(lt, ct, p), k);
-    }
-    return off;
-}
-constexpr int chunk_entries(int lt, bool ct, bool last, int p) {
-    return chunk_offset(lt, ct, last, p, active_stages(lt, ct, p));
-}
-// Chunk stride in entries: a multiple of 16 bytes.
-constexpr int chunk_stride(int lt, bool ct, bool last, int p, int entry_bytes) {
-    const int per16 = 16 / entry_bytes > 0 ? 16 / entry_bytes : 1;
-    const int e = chunk_entries(lt, ct, last, p);
-    return (e + per16 - 1) / per16 * per16;
-}
-// Chunks of one phase: one per block of the stage tree at chunk_shift,
-// over the 2^(prefix_bits + lt) entries the pass covers.
-constexpr std::uint64_t chunk_count(int lt, int prefix_bits, bool ct, int p) {
-    return (std::uint64_t{1} << (prefix_bits + lt)) >> chunk_shift(lt, ct, p);
-}
 
 // Appends one pass's twiddle chunks (piece-major, layout above) to `out` and
 // records each phase's offset from `base`. prefix_bits: 0 for column and
@@ -334,25 +267,6 @@ __device__ __forceinline__ std::uint64_t reduce_wide(std::uint64_t x, const Devi
     const std::uint32_t k = __umulhi(std::uint32_t(x >> 32), std::uint32_t(d.rwp));
     const std::uint64_t p = mad_vs(k, std::uint32_t(d.nq), x);
     return add_high(p, k * std::uint32_t(d.nq >> 32));
-}
-
-// Ranges of the headroom arithmetic, in units of q. Forward: a stage adds 3 to
-// every value; a phase that would pass 16 reduces its values to 3 first.
-// Inverse: sums double, products are 3; see Pass::headroom_stages.
-constexpr int kGrowth = 3, kHeadroomLimit = 16, kReduced = 3;
-constexpr int forward_bound_before(int lt, int p, int bound);
-// Bound after phase p of a forward pass whose values enter below `bound`.
-constexpr int forward_bound_after(int lt, int p, int bound) {
-    const int b = p < 0 ? bound : forward_bound_before(lt, p, bound);
-    return p < 0 ? b : b + kGrowth * active_stages(lt, true, p);
-}
-// Bound entering phase p, after the reduction where it needs one.
-constexpr int forward_bound_before(int lt, int p, int bound) {
-    const int b = forward_bound_after(lt, p - 1, bound);
-    return b + kGrowth * active_stages(lt, true, p) > kHeadroomLimit ? kReduced : b;
-}
-constexpr bool forward_reduces(int lt, int p, int bound) {
-    return forward_bound_after(lt, p - 1, bound) + kGrowth * active_stages(lt, true, p) > kHeadroomLimit;
 }
 
 // Barrett (the constants of the reference's GPU-NTT-compatible provider,
@@ -801,16 +715,13 @@ struct Pass {
         }
     }
 
-    // Bound (in units of q) of the values entering the first pass and, for the
-    // second pass of a forward transform, what the column pass left.
-    static constexpr int kEntry = 4;
-    static constexpr int kForwardEntry =
-        SINGLE || COL ? kEntry : forward_bound_after(L1, num_phases(L1) - 1, kEntry);
-    static constexpr int kForwardExit = forward_bound_after(LT, kPhases - 1, kForwardEntry);
+    // Headroom arithmetic: bounds of the values a forward pass takes in (the second
+    // pass: what the column pass left) and leaves.
+    static constexpr int kForwardEntry = SINGLE || COL ? kHeadroomEntry : forward_exit(L1, kHeadroomEntry);
+    static constexpr int kForwardExit = forward_exit(LT, kForwardEntry);
 
-    // The phase's butterflies in headroom arithmetic. `bound[r]` is v[r]'s range
-    // in units of q: the loops unroll completely, so it is known at compile time
-    // and only the reductions it asks for remain.
+    // The phase's butterflies in headroom arithmetic. The loops unroll completely, so
+    // only the reductions that the schedule asks for remain.
     template <int P>
     static __device__ __forceinline__ void headroom_stages(W (&v)[kE], const Chunk<P>& c, const DeviceDomain<W>& d) {
         constexpr int ws = window_start(LT, CT, P);
@@ -818,13 +729,14 @@ struct Pass {
 #pragma unroll
             for (int r = 0; r < kE; ++r) v[r] = reduce_wide(v[r], d);
         }
+        static_assert(!CT || forward_bound_after(LT, P, kForwardEntry) <= kHeadroomLimit, "forward range");
+        constexpr InversePhase inverse = inverse_phase(LT, CT ? 0 : P, kLast);
+        static_assert(CT || (inverse.pairs_match && inverse.largest <= kHeadroomLimit && inverse.largest_enter <= 6),
+                      "inverse range; spans of 3q and 6q");
         // Multiples of q that keep differences positive, in scalar registers
         // (opaque: the compiler would multiply per butterfly).
-        W q3 = 3 * d.q, q6 = 6 * d.q, q12 = 12 * d.q;
-        asm("" : "+s"(q3), "+s"(q6), "+s"(q12));
-        int bound[kE];
-#pragma unroll
-        for (int r = 0; r < kE; ++r) bound[r] = kReduced;
+        W q3 = 3 * d.q, q6 = 6 * d.q;
+        asm("" : "+s"(q3), "+s"(q6));
 #pragma unroll
         for (int s = 0; s < active_stages(LT, CT, P); ++s) {
             const int k = exec_stage(LT, CT, P, s);
@@ -848,19 +760,14 @@ struct Pass {
                         v[r] = shoup_add(v[r], v[r2], tp, d.nq);
                         v[r2] = twice - v[r];
                     } else {
-                        // Both sides of a pair have the same bound: 3, 6 or 12.
-                        if (bound[r] + bound[r2] > kHeadroomLimit) {
+                        if (inverse.reduce[s][r]) {
                             v[r] = reduce_wide(v[r], d);
                             v[r2] = reduce_wide(v[r2], d);
-                            bound[r] = bound[r2] = kReduced;
                         }
                         const W sum = v[r] + v[r2];
-                        const W span = bound[r2] <= 3 ? q3 : bound[r2] <= 6 ? q6 : q12;
-                        const W diff = v[r] + span - v[r2];
+                        const W diff = v[r] + (inverse.enter[s][r2] <= 3 ? q3 : q6) - v[r2];
                         v[r] = scale ? shoup_add(0, sum, d.ninv, d.nq) : sum;
                         v[r2] = shoup_add(0, diff, scale ? d.last : tp, d.nq);
-                        bound[r] = scale ? kReduced : bound[r] + bound[r2];
-                        bound[r2] = kReduced;
                     }
                 }
             }
@@ -868,7 +775,7 @@ struct Pass {
         if constexpr (!CT) {  // every phase and pass of the inverse starts from kReduced
 #pragma unroll
             for (int r = 0; r < kE; ++r)
-                if (bound[r] > kReduced) v[r] = reduce_wide(v[r], d);
+                if (inverse.reduce_last[r]) v[r] = reduce_wide(v[r], d);
         }
     }
 
