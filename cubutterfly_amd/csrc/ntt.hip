@@ -383,6 +383,7 @@ NttEngine::NttEngine(const NttEngineConfig& c) : impl_(new Impl) {
         .field("output_order", c.output_bit_reversed ? "bit_reversed" : "natural")
         .field("arithmetic", c.barrett ? "barrett" : "shoup")
         .field("lazy_reduction", impl_->u32 ? impl_->u32->lazy : impl_->u64->lazy)
+        .field("headroom", impl_->u64 && impl_->u64->arith == kHeadroom)
         .key("shape")
         .value_raw(impl_->u32 ? impl_->u32->json_shape : impl_->u64->json_shape)
         .field("workspace_bytes", std::uint64_t(workspace_bytes()))

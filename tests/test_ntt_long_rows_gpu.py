@@ -84,6 +84,16 @@ def test_u64_moduli(torch_gpu, lib, stream, kind, log_n, inverse):
     check(torch_gpu, lib, stream, 64, log_n, 3, U64[kind], cb.NttRing.NEGACYCLIC, inverse, False, False)
 
 
+def test_mapping_names_the_arithmetic(torch_gpu, lib):
+    for log_n, batch in ((10, 3), (13, 200), (16, 2)):
+        for kind, q in U64.items():
+            t = cb.describe(cb.Operator.NTT, cb.DataType.UINT64, [1 << log_n], batch, compute=cb.ComputeType.UINT64,
+                            modulus=q, word_bits=64)
+            with cb.Plan(lib, t) as plan:
+                m = plan.mapping()
+                assert m["headroom"] == kind.startswith("headroom") and m["lazy_reduction"] == (kind != "strict")
+
+
 # (256 CUs) The edges of the rule, in natural order: a round half full (u64 2^14:
 # four fifths of one, and no more rounds), two rounds three quarters full; u64 2^13
 # any number of rounds beyond.
