@@ -94,6 +94,20 @@ def test_mapping_names_the_arithmetic(torch_gpu, lib):
                 assert m["headroom"] == kind.startswith("headroom") and m["lazy_reduction"] == (kind != "strict")
 
 
+# Whole rows from natural to bit-reversed order keep the lazy form on the inverse
+# side; the other orders, and two passes, take the one with headroom.
+@pytest.mark.parametrize("log_n", [1, 9, 12, 13])
+@pytest.mark.parametrize("inverse,rin,rout", [(True, False, True), (True, False, False), (False, False, True)])
+def test_staged_inverse_rows_are_lazy(torch_gpu, lib, stream, log_n, inverse, rin, rout):
+    q = U64["headroom-top"]
+    t = cb.describe(cb.Operator.NTT, cb.DataType.UINT64, [1 << log_n], 5, compute=cb.ComputeType.UINT64, modulus=q,
+                    word_bits=64, inverse=inverse, ntt_input_layout=LAYOUT[rin], ntt_output_layout=LAYOUT[rout])
+    with cb.Plan(lib, t) as plan:
+        m = plan.mapping()
+    assert m["lazy_reduction"] and m["headroom"] == (not (inverse and rout and log_n <= 12))
+    check(torch_gpu, lib, stream, 64, log_n, 5, q, cb.NttRing.NEGACYCLIC, inverse, rin, rout)
+
+
 # (256 CUs) The edges of the rule, in natural order: a round half full (u64 2^14:
 # four fifths of one, and no more rounds), two rounds three quarters full; u64 2^13
 # any number of rounds beyond.
