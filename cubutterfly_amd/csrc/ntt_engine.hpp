@@ -76,6 +76,10 @@ class NttEngine {
 // 2^log_n (the `-h<l1>` lowerings), empty elsewhere.
 std::vector<std::uint32_t> ntt_other_splits(std::uint32_t log_n);
 
+// Whether a forward column pass of whole-line tiles leaves an intermediate of
+// `words` words by nontemporal stores, not by write-through ones.
+bool ntt_streams_intermediate(std::uint32_t word_bits, std::uint64_t words);
+
 // Whether moduli in [min_q, max_q] leave four spare bits of a u64 word and have a
 // reciprocal of 32 bits: their lazy butterflies take the headroom form.
 bool ntt_headroom(std::uint32_t word_bits, std::uint64_t min_q, std::uint64_t max_q);

@@ -81,6 +81,7 @@ struct PassArgs {
     const std::uint64_t* out_off;
     std::uint32_t polys, tiles;
     std::uint32_t reduce_input;
+    std::uint32_t stream_out;    // nontemporal intermediate (Pass::kWholeLines)
     std::uint32_t phase_off[4];  // chunk array of each phase, entries from the domain's table start
     std::uint32_t tw_bytes;      // bytes of one domain's chunk tables (buffer range of the twiddle reads)
 };
@@ -432,14 +433,15 @@ struct Pass {
     // inverse, nontemporal / write-through, reused and rotated buffers: u32 2^16 x
     // 64 34.9 / 35.0, 37.9 / 38.8; x 96 53.9 / 46.8, 59.2 / 51.7; x 256 120.6 /
     // 107.3, 134.4 / 116.0; u64 2^16 x 64 72.6 / 72.8, 76.8 / 77.0; x 256 272.5 /
-    // 243.5, 274.2 / 245.1. Only intermediates of 8 MiB lose, in the forward call
-    // by itself (u32 2^16 x 32 10.2 / 10.7, u64 x 16 15.1 / 15.6; with the inverse
-    // after it within 1%). Forward column passes of narrower tiles keep write-back
+    // 243.5, 274.2 / 245.1. Intermediates of a few MiB are the exception and stay
+    // nontemporal (kWholeLines, ntt_streams_intermediate).
+    // Forward column passes of narrower tiles keep write-back
     // stores: write-through made them slower (partial-line segments that the L2
     // would otherwise merge). (Nontemporal final stores measured slower for C4,
     // whose bit-reversed output lands in 8-byte segments: 60.6 -> 71-73 us.)
+    static constexpr bool kWholeLines = COL && CT && !SINGLE && (sizeof(W) << LI) >= 128;
     static constexpr int kStoreAux =
-        !SINGLE && (!CT || (COL ? (sizeof(W) << LI) >= 128 : POUT)) ? 17 : 0;
+        !SINGLE && (!CT || (COL ? kWholeLines : POUT)) ? 17 : 0;
     // A register window starting at tile bit S <= 6 leaves tile bits 10 and up
     // to the wave index (phase_index: thread bits from 6 up are tile bits from
     // 10 up), so an exchange between two such windows never leaves a wave: all
@@ -469,8 +471,7 @@ struct Pass {
     // rotated buffers 38.2 / 38.8 (x 56 37.3 / 38.0, x 40 32.0 / 32.5), other sizes
     // and reused buffers within 1%. u64 tiles lose occupancy for it (2^16 x 32 41.7
     // -> 43.3 us), and one-pass tiles run more waves per SIMD.
-    static constexpr bool kAhead = sizeof(W) == 4 && !SINGLE && !BARRETT && kPhases <= 3 &&
-                                   !(COL && CT && (sizeof(W) << LI) >= 128);
+    static constexpr bool kAhead = sizeof(W) == 4 && !SINGLE && !BARRETT && kPhases <= 3 && !kWholeLines;
 
     // Staged store run: lane l of wave w moves tile elements g0 + 64 kPer k + e
     // (e < kPer), g0 = 1024 w + kPer l. The thread, lane and register parts
@@ -570,10 +571,11 @@ struct Pass {
         if (SINGLE || reg_bytes < 4096u) return buffer_load<W>(src, lane_bytes + reg_bytes);
         return buffer_load<W>(src, lane_bytes, reg_bytes);
     }
+    template <int AUX = kStoreAux>
     static __device__ __forceinline__ void store_at(W x, __amdgpu_buffer_rsrc_t dst, std::uint32_t lane_bytes,
                                                     std::uint32_t reg_bytes) {
-        if (SINGLE || reg_bytes < 4096u) buffer_store<W, kStoreAux>(x, dst, lane_bytes + reg_bytes);
-        else buffer_store<W, kStoreAux>(x, dst, lane_bytes, reg_bytes);
+        if (SINGLE || reg_bytes < 4096u) buffer_store<W, AUX>(x, dst, lane_bytes + reg_bytes);
+        else buffer_store<W, AUX>(x, dst, lane_bytes, reg_bytes);
     }
 
     // Staged (permuted) enumeration: element g of the tile in physical
@@ -919,8 +921,13 @@ struct Pass {
         } else {
             constexpr std::uint32_t B = sizeof(W);
             const std::uint32_t tw = thread_word<wl>(tl, t);
+            if (kWholeLines && a.stream_out) {
 #pragma unroll
-            for (int r = 0; r < kE; ++r) store_at(v[r], dst, tw * B, register_word<wl>(r) * B);
+                for (int r = 0; r < kE; ++r) store_at<2>(v[r], dst, tw * B, register_word<wl>(r) * B);
+            } else {
+#pragma unroll
+                for (int r = 0; r < kE; ++r) store_at(v[r], dst, tw * B, register_word<wl>(r) * B);
+            }
         }
     }
 

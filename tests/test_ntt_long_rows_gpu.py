@@ -108,6 +108,22 @@ def test_staged_inverse_rows_are_lazy(torch_gpu, lib, stream, log_n, inverse, ri
     check(torch_gpu, lib, stream, 64, log_n, 5, q, cb.NttRing.NEGACYCLIC, inverse, rin, rout)
 
 
+# Nontemporal intermediates: u64 2 .. 12 MiB, u32 with 32-column tiles 8 .. 12 MiB,
+# forward only.
+@pytest.mark.parametrize("bits,log_n,batch,inverse,streams", [
+    (64, 16, 3, False, False), (64, 16, 4, False, True), (64, 16, 24, False, True), (64, 16, 25, False, False),
+    (64, 16, 8, True, False), (64, 13, 31, False, False), (64, 13, 32, False, True), (32, 16, 31, False, False),
+    (32, 16, 32, False, True), (32, 16, 48, False, True), (32, 16, 49, False, False), (32, 15, 64, False, False)])
+def test_intermediate_stores(torch_gpu, lib, stream, bits, log_n, batch, inverse, streams):
+    q = U32["lazy"] if bits == 32 else U64["headroom-top"]
+    t = cb.describe(cb.Operator.NTT, cb.DataType.UINT32 if bits == 32 else cb.DataType.UINT64, [1 << log_n], batch,
+                    compute=cb.ComputeType.UINT32 if bits == 32 else cb.ComputeType.UINT64, modulus=q, word_bits=bits,
+                    ntt_ring=cb.NttRing.NEGACYCLIC, inverse=inverse)
+    with cb.Plan(lib, t) as plan:
+        assert plan.mapping()["shape"]["streams_intermediate"] == streams
+    check(torch_gpu, lib, stream, bits, log_n, batch, q, cb.NttRing.NEGACYCLIC, inverse, False, False)
+
+
 # (256 CUs) The edges of the rule, in natural order: a round half full (u64 2^14:
 # four fifths of one, and no more rounds), two rounds three quarters full; u64 2^13
 # any number of rounds beyond.
