@@ -278,10 +278,12 @@ __global__ __launch_bounds__(kThreads) void fwht_columns_kernel(const float* src
 // 20.7; 32 rows with 4 / 1: 5.1 / 3.7, 14.8 / 13.3, 21.8 / 19.6; 16 rows: 3.9 /
 // 3.4, 13.0 / 12.5, 19.0 / 18.4; but 8 rows with 4 / 2: 3.5 / 3.4, 12.2 / 12.5,
 // 17.7 / 18.2. 32 rows from 64 MiB on keep 4 columns, which were as fast there
-// behind the row pass (2^17-point rows: 50.9 / 52.0 us for both passes).
+// behind the row pass (2^17-point rows: 50.9 / 52.0 us for both passes), and 64 rows
+// from 384 MiB on keep 2 (2^18-point rows, both passes, 2 / 1 columns: 256 MiB 176 /
+// 169, 352 255 / 257, 384 280 / 283, 512 379 / 387, 1 GiB 754 / 771).
 template <int LOG_L, bool NARROW>
 constexpr int column_vector() {
-    return NARROW ? (LOG_L <= 5 ? 4 : LOG_L == 6 ? 2 : 1) : LOG_L <= 3 || LOG_L == 5 ? 4 : 1;
+    return NARROW ? (LOG_L <= 5 ? 4 : LOG_L == 6 ? 2 : 1) : LOG_L <= 3 || LOG_L == 5 ? 4 : LOG_L == 6 ? 2 : 1;
 }
 
 // `vec`: the widest vector the pointers' alignment allows.
@@ -291,6 +293,7 @@ void launch_fwht_columns_rows(const float* src, void* dst, std::uint64_t count, 
     constexpr int kVec = column_vector<LOG_L, NARROW>();
     vec = std::min(vec, kVec);
     if (!NARROW && LOG_L == 5 && count < (std::uint64_t{1} << 24)) vec = 1;
+    if (!NARROW && LOG_L == 6 && count < (std::uint64_t{3} << 25)) vec = 1;
     const std::uint64_t vectors = count >> (LOG_L + (vec == 4 ? 2 : vec == 2 ? 1 : 0));
     const std::uint64_t blocks = (vectors + kThreads - 1) / kThreads;
     require(blocks < (std::uint64_t{1} << 31), "FWHT column pass grid too large");

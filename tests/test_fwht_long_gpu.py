@@ -29,6 +29,26 @@ def test_forward_bit_exact(torch_gpu, lib, stream, log_n, batch):
     np.testing.assert_array_equal(got.view(np.uint32), expected.view(np.uint32))
 
 
+def test_column_pass_width_by_size(torch_gpu, lib, stream):
+    # From 384 MiB on a lane of the 64-row column pass holds two columns, below
+    # one: the whole batch equals its halves bit for bit, and the oracle.
+    log_n, batch = 18, 384
+    x = torch_gpu.randn((batch, 1 << log_n), device="cuda", generator=torch_gpu.Generator("cuda").manual_seed(9))
+    outs = []
+    for rows in (batch, batch // 2):
+        y = torch_gpu.empty_like(x)
+        with cb.Plan(lib, fwht(1 << log_n, rows), stream=stream) as plan:
+            assert plan.workspace_size() == 0
+            for first in range(0, batch, rows):
+                plan.execute(x[first:first + rows], y[first:first + rows])
+            torch_gpu.cuda.synchronize()
+        outs.append(y)
+    assert torch_gpu.equal(outs[0].view(torch_gpu.int32), outs[1].view(torch_gpu.int32))
+    rows = [0, 191, 192, 383]
+    expected = oracle.fwht_f32(x[rows].cpu().numpy(), threads=oracle.default_threads())
+    np.testing.assert_array_equal(outs[0][rows].cpu().numpy().view(np.uint32), expected.view(np.uint32))
+
+
 def test_inverse_normalised_and_in_place(torch_gpu, lib, stream):
     x = np.random.default_rng(3).standard_normal((3, 1 << 16)).astype(np.float32)
     got = run_plan(torch_gpu, lib, fwht(1 << 16, 3, inverse=True, placement=cb.Placement.IN_PLACE), x, stream, in_place=True)
