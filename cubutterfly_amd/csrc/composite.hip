@@ -15,10 +15,11 @@
 // stored transposed, then the rows of the transposed block, stored back in
 // the original order (two HBM round trips where the transposes take four).
 // The transposing store writes segments of 2^(14 - n) elements for rows of
-// 2^n points; where an axis has 2^11 points or more (segments under 128
-// bytes), or axis 0 2^9 in 2^21 points or more, the block runs instead as column
-// passes over axis 0 and a row pass over axis 1 that stores whole rows (the
-// exceptions stand at the rule in CompositeExecutor). Blocks of
+// 2^n points (128 bytes at 2^9 and 64 at 2^10, whose tiles are half as large;
+// 64 and 32 at 2^11 and 2^12). Where an axis has 2^11 points or more, or axis 0
+// 2^9 in 2^21 points or more, the block runs instead as column passes over axis
+// 0 and a row pass over axis 1 that stores whole rows (the exceptions and the
+// figures stand at the rule in CompositeExecutor). Blocks of
 // at most 2^14 points are transformed whole, both axes in one pass. Each lowering
 // can be named (EXPLICIT) where its kernels cover the shape.
 //

@@ -975,9 +975,9 @@ void add() {
 // Shapes: one pass for m <= 14 (2^12-point tiles, 2^13 / 2^14 for m = 13,
 // 14); two passes with 2^14-point tiles (2^13 for some 9- and 10-bit passes,
 // below) over l1 = m / 2 high bits (column
-// tiles) and l2 = m - l1 low bits (row tiles). The even split keeps both the
-// column reads and the transposing row stores in segments of 2^(14 - m/2)
-// elements (32 bytes at m = 24); a column-heavier split would leave the
+// tiles) and l2 = m - l1 low bits (row tiles). The even split keeps the column
+// reads and the transposing row stores in segments of similar length, col_lines
+// and row_lines (32 bytes at m = 24); a column-heavier split would leave the
 // transposing store with single-element segments.
 constexpr int single_li(int m) { return m < 12 ? 12 - m : 0; }
 constexpr int split_l1(int m) { return m / 2; }
@@ -1007,11 +1007,10 @@ void add_two() {
     add<l2, row_lines(l1, l2), false, false>();
 }
 
-// Row passes over natural-order rows with the transposing store, tiles of
-// 2^14 points (2^(14 - LT) rows, at least 4 so the transposed segments are
-// 32 bytes or longer).
-// Rank-2 row passes with a transposing store: likewise (512 x 512 blocks, 2^19
-// points, both passes 22.2 / 14.6 us, 2^23 65.8 / 57.0).
+// Row passes over natural-order rows with the transposing store: tiles of 2^14
+// points, 2^13 for rows of 9 and 10 bits (as in the passes above: 512 x 512 blocks,
+// 2^19 points, both passes 22.2 / 14.6 us, 2^23 65.8 / 57.0), at least 4 rows so
+// the transposed segments are 32 bytes or longer.
 constexpr int transposed_lines(int l2) { return l2 == 9 || l2 == 10 ? 13 - l2 : 14 - l2; }
 template <int LT>
 void add_rows_natural() {
@@ -1020,8 +1019,8 @@ void add_rows_natural() {
     registry()[Key{LT, li, false, false, true, 4}] = &launch<LT, li, false, false, true, 4>;
 }
 
-// Rank-2 blocks: column passes of 2^LT points over whole 2^14-point tiles,
-// and rows written back in natural order in 2^12-point tiles (a quarter of
+// Rank-2 blocks: column passes of 2^LT points over tiles of whole row segments
+// (rank2_column_lines), and rows written back in natural order in 2^12-point tiles (a quarter of
 // the LDS each, so four workgroups per CU overlap one another's loads and
 // butterflies where the rows of 2^9 points and more have no prefetching walk).
 template <int LT>
@@ -1150,7 +1149,7 @@ int parse_split(int m, const std::string& name) {
 // batched 2^(b + c)-point transforms over the middle b bits (its level
 // twiddles are those of the full transform: a DIF digit's twiddle depends
 // only on the bits below it), and the row pass of a (a + b) x c split. Every
-// pass moves segments of 2^min(14 - bits, ...) elements (512 bytes at
+// pass moves segments of 2^col_lines or 2^row_lines elements (512 bytes at
 // 8 + 8 + 8), where the two-pass 12 + 12 split moves 32-byte segments.
 bool split3_available(int m, int a, int b, bool inverse, int ord = 0) {
     const int c = m - a - b;
@@ -1619,8 +1618,9 @@ class FftRank2BlocksExecutor final : public Executor {
 // independent transforms, FftArgs::cbits), then the rows: each row pass tile
 // gathers rows from the column passes' bit-reversed axis-0 order and writes
 // them back transformed, in natural order. Every pass reads and writes whole
-// segments of 2^(14 - t) columns or whole rows, where the transposing row
-// passes of the same blocks move 2^(14 - l1)-element segments.
+// segments of columns (2^rank2_column_lines(t) in a first pass of t bits, 2^(14 - t)
+// in a second one) or whole rows, where the transposing row passes of the same
+// blocks move segments of 2^transposed_lines(l1) elements.
 class FftRank2ColumnsExecutor final : public Executor {
   public:
     FftRank2ColumnsExecutor(const Request& r, std::uint32_t l0, std::uint32_t ta, std::uint32_t tb) {
@@ -1737,15 +1737,16 @@ std::unique_ptr<Executor> make_fft_rows_transposed(const Request& r, std::uint32
 
 // The column-pass split of axis 0 (ta top bits, then tb; tb = 0 for one
 // pass), or false where no kernels cover the shape: rows of 2^5 .. 2^12
-// points (whole 2^14-point column tiles within a block), blocks of at most 2^24
+// points (whole column tiles within a block), blocks of at most 2^24
 // points (the level-twiddle tables' reach), and axis 0 in one column pass of
 // 4 .. 11 bits, its tile's columns within the 2^l1 of a row, or two: the
 // second over tb >= 14 - l1 bits, the first over the rest, each within 4 .. 8
 // bits. One pass of 9 to 11 bits moves segments of 128 or 64 bytes and still
 // beats two (2^23 points, 2048 x 1024: 53.8 against 74.7 us, 2048 x 2048 53.5
-// against 76.1). Blocks with 2^12-point rows keep two from 2^9 points on,
-// though one is faster there too (512 x 4096 x 2 50.4 / 33.3 us, 2048 x 4096 78.0
-// / 58.9): their mapping (`column_passes`) is what programs have seen.
+// against 76.1). Blocks with 2^12-point rows still take two from 2^9 points on,
+// the split they had before single passes of 9 to 11 bits existed, and which
+// tests/test_composite_gpu.py pins. That is not the faster one (512 x 4096 x 2: two
+// 50.4, one 33.3 us; 2048 x 4096: 78.0, 58.9).
 bool rank2_columns_split(const Request& r, std::uint32_t l0, std::uint32_t& ta, std::uint32_t& tb) {
     const std::uint32_t m = r.log_n;
     if (l0 < 4 || l0 >= m) return false;
