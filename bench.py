@@ -214,7 +214,7 @@ class FwhtFp32Pitched(FwhtFp32):
 class NttNegacyclic(Workload):
     """C2: forward then inverse negacyclic NTT, u32, q = 1073479681, n = 2^16, batch 64."""
     name, dtype = "c2", "u32"
-    valu_per_butterfly = 8.6
+    valu_per_butterfly = 8.7
 
     def __init__(self, log_n=16, batch=64):
         from cubutterfly_amd import workloads
@@ -269,7 +269,7 @@ class RnsNegacyclic(Workload):
     name, dtype = "c4", "u64"
     description = ("C4: RNS negacyclic NTT u64, n=2^16, 32 limbs of distinct 60-bit primes (q = 1 mod 2^17), "
                    "one step = forward (natural->bit_reversed) then inverse (bit_reversed->natural)")
-    valu_per_butterfly = 26.1
+    valu_per_butterfly = 19.2
     takes_mapping = False
 
     def __init__(self, log_n=16, limbs=32):

@@ -90,9 +90,11 @@ __device__ __forceinline__ void exchange(float (&v)[kE], float* lds, unsigned t)
 // ---- storage adapters ----------------------------------------------------
 
 // FP32 results stored straight from the last phase (one element per lane,
-// a wave covering 256 consecutive bytes) use nontemporal stores: each output
-// is written once and not read again, and C1 measured 25.7 -> 20.9 us on
-// MI355X. So do the 32-register kernel's runs (wide_store_run). The
+// a wave covering 256 consecutive bytes) use nontemporal stores: a one-pass
+// plan writes each output once and does not read it again, and C1 measured 25.7
+// -> 20.9 us on MI355X. (The rows of a factored plan, which a column pass reads
+// back, leave the same way; no other policy was measured there.) So do the
+// 32-register kernel's runs (wide_store_run). The
 // 16-register kernel's 16-byte vector stores, 32 bytes apart across the
 // lanes, keep the default policy, where the hint measured slower (C5b 50.2
 // -> 55.3 us; regrouped through LDS into 1 KiB per wave instruction, 51.7-
