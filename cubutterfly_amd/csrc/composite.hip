@@ -271,30 +271,33 @@ __global__ __launch_bounds__(kThreads) void fwht_columns_kernel(const float* src
     }
 }
 
-// Consecutive columns per lane: up to 4 of at most 8 rows, one of more (FP16
-// results: as many as the registers hold, so a lane's halves make whole words).
-// A pass is bound by the loads in flight, and one column of 16 or more rows per
-// lane means more waves: the pass alone, FP32 rows of 2^18 points, 64 rows with
+// Consecutive columns per lane: as many as the registers hold, up to 4 (FP16 results:
+// so a lane's halves make whole words), but one of 16 to 64 rows. A pass is bound by
+// the loads in flight, and one column per lane means more waves: the pass alone, FP32
+// rows of 2^18 points, 64 rows with
 // 2 / 1 columns a lane: 8 MiB 6.9 / 4.5 us, 40 MiB 17.6 / 13.7, 64 MiB 21.6 /
 // 20.7; 32 rows with 4 / 1: 5.1 / 3.7, 14.8 / 13.3, 21.8 / 19.6; 16 rows: 3.9 /
 // 3.4, 13.0 / 12.5, 19.0 / 18.4; but 8 rows with 4 / 2: 3.5 / 3.4, 12.2 / 12.5,
-// 17.7 / 18.2. 32 rows from 64 MiB on keep 4 columns, which were as fast there
-// behind the row pass (2^17-point rows: 50.9 / 52.0 us for both passes), and 64 rows
-// from 384 MiB on keep 2 (2^18-point rows, both passes, 2 / 1 columns: 256 MiB 176 /
-// 169, 352 255 / 257, 384 280 / 283, 512 379 / 387, 1 GiB 754 / 771).
-template <int LOG_L, bool NARROW>
+// 17.7 / 18.2. Three exceptions:
+//  - 32 rows from 64 MiB on keep 4 columns, as fast there behind the row pass
+//    (2^17-point rows: 50.9 / 52.0 us for both passes);
+//  - 64 rows from 384 MiB on keep 2 (2^18-point rows, both passes, 2 / 1 columns: 256
+//    MiB 176 / 169, 352 255 / 257, 384 280 / 283, 512 379 / 387, 1 GiB 754 / 771);
+//  - `wide`: all passes of a transform of several (wide_columns).
+template <int LOG_L>
 constexpr int column_vector() {
-    return NARROW ? (LOG_L <= 5 ? 4 : LOG_L == 6 ? 2 : 1) : LOG_L <= 3 || LOG_L == 5 ? 4 : LOG_L == 6 ? 2 : 1;
+    return LOG_L <= 5 ? 4 : LOG_L == 6 ? 2 : 1;
 }
 
 // `vec`: the widest vector the pointers' alignment allows.
 template <int LOG_L, bool NARROW>
 void launch_fwht_columns_rows(const float* src, void* dst, std::uint64_t count, std::uint32_t log_cols, int vec,
-                              float scale, bool apply_scale, float out_scale, hipStream_t stream) {
-    constexpr int kVec = column_vector<LOG_L, NARROW>();
+                              bool wide, float scale, bool apply_scale, float out_scale, hipStream_t stream) {
+    constexpr int kVec = column_vector<LOG_L>();
     vec = std::min(vec, kVec);
-    if (!NARROW && LOG_L == 5 && count < (std::uint64_t{1} << 24)) vec = 1;
-    if (!NARROW && LOG_L == 6 && count < (std::uint64_t{3} << 25)) vec = 1;
+    if (!NARROW && LOG_L >= 4 && !wide && (LOG_L != 5 || count < (std::uint64_t{1} << 24)) &&
+        (LOG_L != 6 || count < (std::uint64_t{3} << 25)))
+        vec = 1;
     const std::uint64_t vectors = count >> (LOG_L + (vec == 4 ? 2 : vec == 2 ? 1 : 0));
     const std::uint64_t blocks = (vectors + kThreads - 1) / kThreads;
     require(blocks < (std::uint64_t{1} << 31), "FWHT column pass grid too large");
@@ -319,24 +322,25 @@ void launch_fwht_columns_rows(const float* src, void* dst, std::uint64_t count, 
 
 template <bool NARROW>
 void launch_fwht_columns_of(const float* src, void* dst, std::uint64_t count, std::uint32_t log_rows,
-                            std::uint32_t log_cols, int vec, float scale, bool apply_scale, float out_scale,
-                            hipStream_t stream) {
+                            std::uint32_t log_cols, int vec, bool wide, float scale, bool apply_scale,
+                            float out_scale, hipStream_t stream) {
     switch (log_rows) {
-        case 1: launch_fwht_columns_rows<1, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
-        case 2: launch_fwht_columns_rows<2, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
-        case 3: launch_fwht_columns_rows<3, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
-        case 4: launch_fwht_columns_rows<4, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
-        case 5: launch_fwht_columns_rows<5, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
-        case 6: launch_fwht_columns_rows<6, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
-        default: launch_fwht_columns_rows<7, NARROW>(src, dst, count, log_cols, vec, scale, apply_scale, out_scale, stream); break;
+        case 1: launch_fwht_columns_rows<1, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
+        case 2: launch_fwht_columns_rows<2, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
+        case 3: launch_fwht_columns_rows<3, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
+        case 4: launch_fwht_columns_rows<4, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
+        case 5: launch_fwht_columns_rows<5, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
+        case 6: launch_fwht_columns_rows<6, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
+        default: launch_fwht_columns_rows<7, NARROW>(src, dst, count, log_cols, vec, wide, scale, apply_scale, out_scale, stream); break;
     }
 }
 
 // Column pass over `count` FP32 elements (G blocks of 2^log_rows x
 // 2^log_cols), src == dst allowed; with `narrow_out`, the results go there as
-// FP16 (narrow_scaled(x, out_scale)) instead.
+// FP16 (narrow_scaled(x, out_scale)) instead. `wide`: see
+// wide_columns.
 void launch_fwht_columns(const float* src, float* dst, std::uint64_t count, std::uint32_t log_rows,
-                         std::uint32_t log_cols, float scale, bool apply_scale, hipStream_t stream,
+                         std::uint32_t log_cols, bool wide, float scale, bool apply_scale, hipStream_t stream,
                          __half* narrow_out = nullptr, float out_scale = 1.0f) {
     require(log_rows >= 1 && log_rows <= kMaxColumnBits && log_cols >= 6, "FWHT column pass shape");
     const auto s = reinterpret_cast<std::uintptr_t>(src);
@@ -349,10 +353,11 @@ void launch_fwht_columns(const float* src, float* dst, std::uint64_t count, std:
         vec = std::min(vec, d % 16 == 0 ? 4 : d % 8 == 0 ? 2 : 1);
     }
     if (narrow_out)
-        launch_fwht_columns_of<true>(src, narrow_out, count, log_rows, log_cols, vec, scale, apply_scale, out_scale,
-                                     stream);
+        launch_fwht_columns_of<true>(src, narrow_out, count, log_rows, log_cols, vec, wide, scale, apply_scale,
+                                     out_scale, stream);
     else
-        launch_fwht_columns_of<false>(src, dst, count, log_rows, log_cols, vec, scale, apply_scale, 1.0f, stream);
+        launch_fwht_columns_of<false>(src, dst, count, log_rows, log_cols, vec, wide, scale, apply_scale, 1.0f,
+                                      stream);
     hip_check(hipGetLastError(), "FWHT column pass launch");
 }
 
@@ -368,6 +373,32 @@ struct Step {
     bool apply_scale = false;             // columns: times `scale` after the stages
     float scale = 1.0f;
 };
+
+// Whether all column passes of a transform of `count` elements hold as many columns
+// per lane as the registers allow. Passes of 16 and 32 rows do where there are several
+// and the data is about what the L2s hold; one choice for all, since a pass that
+// spreads the data over the workgroups in another way than the one before it finds
+// less of it in its L2 ([16, 16, 64], 12 MiB: 22.2 wide, 23.1 narrow, 25.9 us mixed).
+// Whole inverses, wide / narrow: [256, 256] 12 MiB 25.7 / 24.7, 16 29.7 / 30.7, 20 29.8
+// / 31.2, 32 38.8 / 39.7, 48 55.4 / 54.2; [16, 16, 64] 8 MiB 17.2 / 17.3, 12 22.2 /
+// 23.1, 16 23.4 / 29.1, 32 36.0 / 39.0, 48 55.0 / 53.8; with 32 rows, on rotated
+// buffers, [512, 128] 14 MiB 27.7 / 27.8, 16 27.9 / 29.1, 28 36.7 / 36.4, [16, 32, 128]
+// 14 27.4 / 26.7, 16 27.8 / 28.5, 20 30.9 / 30.2. 64 rows are narrow at each of these
+// sizes ([4096, 128] 16 MiB 35.3 / 31.3).
+bool wide_columns(const std::vector<Step>& steps, std::uint64_t count) {
+    int passes = 0;
+    std::uint32_t most_rows = 0, least_cols = 64;
+    for (const Step& s : steps)
+        if (s.columns) {
+            ++passes;
+            most_rows = std::max(most_rows, s.log_rows);
+            least_cols = std::min(least_cols, s.log_cols);
+        }
+    const std::uint64_t mi = std::uint64_t{1} << 20;
+    if (passes < 2 || most_rows > 5) return false;
+    return most_rows <= 4 ? count > (least_cols < 8 ? 2 : 3) * mi && count <= 10 * mi
+                          : 2 * count > 7 * mi && 2 * count <= 9 * mi;
+}
 
 class CompositeExecutor final : public Executor {
   public:
@@ -525,6 +556,7 @@ class CompositeExecutor final : public Executor {
             for (std::uint32_t axis = 0; axis < rank; ++axis) move_innermost(axis);
         }
         if (rank == 1 && r.embedding && !flatten && r.op == Op::Fft) ragged_ = use_ragged_rows();
+        wide_ = wide_columns(steps_, r.n * r.batch);
         for (const auto& c : children_) {
             if (!fwht_columns_) names.push_back(c->algorithm);
             child_ws_ = std::max(child_ws_, c->workspace_bytes());
@@ -683,7 +715,7 @@ class CompositeExecutor final : public Executor {
                 require(cur_writable != nullptr, "an FWHT column pass runs on a step's destination");
                 const bool narrow_here = narrow != nullptr && i + 1 == steps_.size();
                 launch_fwht_columns(static_cast<const float*>(cur_writable), static_cast<float*>(cur_writable),
-                                    count, s.log_rows, s.log_cols, s.scale, s.apply_scale, stream,
+                                    count, s.log_rows, s.log_cols, wide_, s.scale, s.apply_scale, stream,
                                     narrow_here ? narrow : nullptr, out_scale);
                 continue;
             }
@@ -816,6 +848,7 @@ class CompositeExecutor final : public Executor {
     Request r_;
     bool transposing_ = false, columns_ = false, blocks_ = false, fwht_columns_ = false;
     bool ragged_ = false;  // the child reads and writes the caller's rows (rank-1 embedding)
+    bool wide_ = false;    // wide_columns
     bool direct_in_ = false, direct_out_ = false;
     NdSide in_side_, out_side_;
     std::vector<std::unique_ptr<Executor>> children_;

@@ -49,6 +49,21 @@ def test_column_pass_width_by_size(torch_gpu, lib, stream):
     np.testing.assert_array_equal(outs[0][rows].cpu().numpy().view(np.uint32), expected.view(np.uint32))
 
 
+# Column passes of 16 and 32 rows at the edges of their widths by size (12 and 40
+# MiB, 8 MiB of 64 columns, 18 MiB with 32 rows): bit for bit.
+@pytest.mark.parametrize("extents,batch", [((256, 256), 48), ((256, 256), 49), ((256, 256), 160), ((256, 256), 161),
+                                           ((16, 16, 64), 128), ((16, 16, 64), 129), ((512, 128), 72), ((512, 128), 73),
+                                           ((16, 256), 769)])
+def test_column_widths_of_several_passes(torch_gpu, lib, stream, extents, batch):
+    n = int(np.prod(extents))
+    x = np.random.default_rng(batch).standard_normal((batch, n)).astype(np.float32)
+    t = cb.describe(cb.Operator.FWHT, cb.DataType.FP32, list(extents), compute=cb.ComputeType.FP32, batch=batch,
+                    inverse=True)
+    got = run_plan(torch_gpu, lib, t, x, stream).reshape(batch, n)
+    want = oracle.fwht_f32(x, inverse=True, normalize=True, threads=oracle.default_threads())
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_inverse_normalised_and_in_place(torch_gpu, lib, stream):
     x = np.random.default_rng(3).standard_normal((3, 1 << 16)).astype(np.float32)
     got = run_plan(torch_gpu, lib, fwht(1 << 16, 3, inverse=True, placement=cb.Placement.IN_PLACE), x, stream, in_place=True)
