@@ -140,15 +140,17 @@ struct EngineImplT {
         lazy = !c.force_strict && !c.barrett && max_q < (std::uint64_t{1} << (bits - 2));
         supported(!c.barrett || max_q < (std::uint64_t{1} << (bits - 2)),
                   "Barrett arithmetic needs every modulus below 2^" + std::to_string(bits - 2));
-        // Whole rows of up to 2^12 points, inverse from natural to bit-reversed order,
-        // keep the lazy form: with both boundaries LDS-staged the headroom kernels take
-        // 138 registers (118), three waves per SIMD in place of four (2^12 x 1024 33.2 /
-        // 30.8 us, x 2048 56.6 / 53.4), and compiled for four they spill (2^10 x 16384
-        // 88 / 78).
-        const bool staged_rows = c.inverse && log_n <= 12 && !c.input_bit_reversed && c.output_bit_reversed;
+        const std::uint64_t polys = c.polynomials.empty() ? c.batch : c.polynomials.size();
+        // Rows of 2^12 points, inverse from natural to bit-reversed order, keep the lazy
+        // form where more than two per CU run: with both boundaries LDS-staged the
+        // headroom kernel takes 138 registers (118), three workgroups per CU in place of
+        // four (headroom / lazy: x 256 13.7 / 14.2 us, 512 19.9 / 19.9, 1024 33.1 / 30.6,
+        // 2048 56.7 / 54.5, 4096 102.8 / 95.5; compiled for four it spills and is slower
+        // still). Shorter rows do not lose.
+        const bool staged_rows = c.inverse && log_n == 12 && !c.input_bit_reversed && c.output_bit_reversed &&
+                                 polys > 2 * std::uint64_t(device_cu_count());
         const bool headroom = lazy && !staged_rows && ntt_headroom(bits, min_q, max_q);
         arith = c.barrett ? kBarrett : headroom ? kHeadroom : lazy ? kLazy : kStrict;
-        const std::uint64_t polys = c.polynomials.empty() ? c.batch : c.polynomials.size();
         require(polys >= 1 && polys <= 0xffffffffull, "NTT batch must be in [1, 2^32)");
         const bool offsets = !c.polynomials.empty();
         PassArgs<W> in_args{}, out_args{};  // the caller's sides: offsets of the first and last pass

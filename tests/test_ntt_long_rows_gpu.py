@@ -94,18 +94,19 @@ def test_mapping_names_the_arithmetic(torch_gpu, lib):
                 assert m["headroom"] == kind.startswith("headroom") and m["lazy_reduction"] == (kind != "strict")
 
 
-# Whole rows from natural to bit-reversed order keep the lazy form on the inverse
-# side; the other orders, and two passes, take the one with headroom.
-@pytest.mark.parametrize("log_n", [1, 9, 12, 13])
-@pytest.mark.parametrize("inverse,rin,rout", [(True, False, True), (True, False, False), (False, False, True)])
-def test_staged_inverse_rows_are_lazy(torch_gpu, lib, stream, log_n, inverse, rin, rout):
+# (256 CUs) More than two 2^12-point rows per CU, inverse from natural to bit-reversed
+# order, keep the lazy form; fewer, shorter ones and other orders take headroom.
+@pytest.mark.parametrize("log_n,batch,inverse,rin,rout", [(12, 512, True, False, True), (12, 513, True, False, True),
+                                                          (11, 1025, True, False, True), (12, 513, True, False, False),
+                                                          (12, 513, False, False, True), (1, 5, True, False, True)])
+def test_staged_inverse_rows_are_lazy(torch_gpu, lib, stream, log_n, batch, inverse, rin, rout):
     q = U64["headroom-top"]
-    t = cb.describe(cb.Operator.NTT, cb.DataType.UINT64, [1 << log_n], 5, compute=cb.ComputeType.UINT64, modulus=q,
+    t = cb.describe(cb.Operator.NTT, cb.DataType.UINT64, [1 << log_n], batch, compute=cb.ComputeType.UINT64, modulus=q,
                     word_bits=64, inverse=inverse, ntt_input_layout=LAYOUT[rin], ntt_output_layout=LAYOUT[rout])
     with cb.Plan(lib, t) as plan:
         m = plan.mapping()
-    assert m["lazy_reduction"] and m["headroom"] == (not (inverse and rout and log_n <= 12))
-    check(torch_gpu, lib, stream, 64, log_n, 5, q, cb.NttRing.NEGACYCLIC, inverse, rin, rout)
+    assert m["lazy_reduction"] and m["headroom"] == (not (inverse and rout and log_n == 12 and batch > 512))
+    check(torch_gpu, lib, stream, 64, log_n, batch, q, cb.NttRing.NEGACYCLIC, inverse, rin, rout)
 
 
 # Nontemporal intermediates: u64 2 .. 12 MiB, u32 with 32-column tiles 8 .. 12 MiB,
