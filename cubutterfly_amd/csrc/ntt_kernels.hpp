@@ -960,7 +960,8 @@ struct Pass {
         // every line at once: fetched one after another as their fields came up, they
         // had cost small batches 3% (u64, q of 63 bits, forward / inverse alone:
         // 2^13 x 16 12.2 / 13.2 -> 11.7 / 12.9 us).
-        asm volatile("" ::"s"(a.domain.q), "s"(a.domain.tw), "s"(a.in_off), "s"(a.tw_bytes));
+        // (One-pass kernels, whose rows wait longer for their loads, gain nothing.)
+        if constexpr (!SINGLE) asm volatile("" ::"s"(a.domain.q), "s"(a.domain.tw), "s"(a.in_off), "s"(a.tw_bytes));
         const std::uint32_t b = blockIdx.x;
         // XCD-contiguous tile order: blocks are dealt to the 8 XCDs
         // round-robin, so block b walks tile (b mod 8) * tiles/8 + b/8 and the
