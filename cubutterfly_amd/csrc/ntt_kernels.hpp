@@ -964,10 +964,10 @@ struct Pass {
         if constexpr (!SINGLE) asm volatile("" ::"s"(a.domain.q), "s"(a.domain.tw), "s"(a.in_off), "s"(a.tw_bytes));
         const std::uint32_t b = blockIdx.x;
         // XCD-contiguous tile order: blocks are dealt to the 8 XCDs
-        // round-robin, so block b walks tile (b mod 8) * tiles/8 + b/8 and the
-        // tiles sharing cache lines and twiddle rows meet in one L2.
-        const std::uint32_t index =
-            (a.tiles & 7u) == 0 && (gridDim.x & 7u) == 0 ? (b & 7u) * (a.tiles >> 3) + (b >> 3) : b;
+        // round-robin, so block b walks tile b/8 of the (b mod 8)-th eighth (one tile
+        // more in the first tiles mod 8 of them), and the tiles sharing cache lines and
+        // twiddle rows meet in one L2.
+        const std::uint32_t xcd = b & 7u, index = xcd * (a.tiles >> 3) + min(xcd, a.tiles & 7u) + (b >> 3);
         tile(a, index, lds);
     }
 };

@@ -109,6 +109,15 @@ def test_staged_inverse_rows_are_lazy(torch_gpu, lib, stream, log_n, batch, inve
     check(torch_gpu, lib, stream, 64, log_n, batch, q, cb.NttRing.NEGACYCLIC, inverse, rin, rout)
 
 
+# Tile counts that no multiple of 8 divides: every tile is some block's.
+@pytest.mark.parametrize("bits,log_n,batch", [(64, 13, 1), (64, 13, 7), (64, 16, 3), (32, 14, 157), (32, 10, 29), (64, 12, 9),
+                                              (32, 15, 1)])
+def test_odd_tile_counts(torch_gpu, lib, stream, bits, log_n, batch):
+    q = U32["lazy"] if bits == 32 else U64["headroom-top"]
+    for inverse in (False, True):
+        check(torch_gpu, lib, stream, bits, log_n, batch, q, cb.NttRing.NEGACYCLIC, inverse, False, False)
+
+
 # Nontemporal intermediates: u64 2 .. 12 MiB, u32 with 32-column tiles 8 .. 12 MiB,
 # forward only.
 @pytest.mark.parametrize("bits,log_n,batch,inverse,streams", [
